@@ -1,0 +1,513 @@
+"""The workloads this framework is timed on: draws of the exact leverage
+sampler, sampler construction, sampled and exact CP-ALS updates, the
+Larsen-Kolda sampler and the draw server, through the package's public classes.
+
+A case is a dict of plain values.  ``listed()`` gives the fixed ones, ``draw``
+further ones of the same ranges; ``prepare`` builds what a program holds before
+the call, ``run`` is one pass, ``work`` the bytes and operations a pass cannot
+do without, and ``exact`` the result in 64 bits by brute force (row scans and
+dense eigendecompositions, none of the package's code)."""
+import math
+
+import numpy as np
+import torch
+
+import fast_tensor_leverage_amd as ftl
+
+DEV = "cuda"
+BRUTE_LIMIT = 2.5e11  # sample x row products exact() goes through at most
+
+
+# --------------------------------------------------------------------------- cases
+def listed():
+    return [
+        # the reference's small exact-sampler configuration, through the NumPy
+        # interface a switched script calls: latency and launches
+        {"name": "draw_host_small", "op": "draw_host", "dims": "1000x1000x1000x1000", "R": 8, "J": 10000, "j": 5,
+         "precision": "fp64", "factors": "gauss"},
+        # the headline: 2^69 KRP rows, every mode, FP32 trees, caller's uniforms
+        {"name": "draw_fp32_headline", "op": "draw", "dims": "8388608x8388608x8388608", "R": 32, "J": 50000, "j": 4,
+         "precision": "fp32", "factors": "gauss", "uniforms": "given"},
+        # the plain FP64 sampler with one mode excluded (an ALS solve's draw)
+        {"name": "draw_fp64_exclude", "op": "draw", "dims": "4194304x4194304x4194304", "R": 32, "J": 50000, "j": 1,
+         "precision": "fp64", "factors": "gauss", "uniforms": "builtin"},
+        # large rank on ill-conditioned factors (mixed precision)
+        {"name": "draw_fp32_r128", "op": "draw", "dims": "1048576x1048576x1048576", "R": 128, "J": 50000, "j": 4,
+         "precision": "fp32", "factors": "graded", "uniforms": "given"},
+        # uneven odd sizes at R = 64, fewer samples
+        {"name": "draw_fp64_r64_ragged", "op": "draw", "dims": "300007x70001x1500017", "R": 64, "J": 20011, "j": 4,
+         "precision": "fp64", "factors": "gauss", "uniforms": "given"},
+        # many modes, small rank
+        {"name": "draw_fp32_n6_r16", "op": "draw", "dims": "262144x131071x262144x65537x262144x200000", "R": 16,
+         "J": 65536, "j": 7, "precision": "fp32", "factors": "gauss", "uniforms": "builtin"},
+        # new factors: the sampler built from device factors, then drawn from
+        {"name": "build_draw_fp64", "op": "build", "dims": "2097152x2097152x2097152", "R": 32, "J": 8192, "j": 4,
+         "precision": "fp64", "factors": "gauss", "uniforms": "given"},
+        # sampled CP-ALS sweep on a 4-way tensor of short modes (the shape of
+        # FROSTT's Uber), factors kept in NumPy as in the reference
+        {"name": "als_sweep_uber", "op": "als", "dims": "183x24x1140x1717", "nnz": 3309490, "R": 25, "J": 65536,
+         "host_sync": True},
+        # sampled CP-ALS sweep on a long 3-way tensor, factors on the device
+        {"name": "als_sweep_long", "op": "als", "dims": "1048576x524288x32768", "nnz": 20000000, "R": 25, "J": 65536,
+         "host_sync": False},
+        # exact CP-ALS sweep and the fit's residual
+        {"name": "als_exact", "op": "als_exact", "dims": "65536x32768x4096", "nnz": 2000000, "R": 25},
+        # Larsen-Kolda: rescore one factor, draw
+        {"name": "larsen_kolda", "op": "lk", "dims": "1048576x524288x300007", "R": 32, "J": 50000, "j": 4},
+        # a burst of requests on resident factor sets and on new ones
+        {"name": "serve_burst", "op": "serve", "shapes": 3, "sets": 6, "on_sets": 24, "fresh": 8, "max_log2_rows": 20,
+         "precision": "fp32"},
+    ]
+
+
+def _size(rng, lo, hi):
+    v = int(round(2 ** rng.uniform(math.log2(lo), math.log2(hi))))
+    return v | 1 if rng.random() < 0.5 else v
+
+
+def draw(rng):
+    op = rng.choice(["draw"] * 6 + ["draw_host", "build", "build", "als", "als", "als_exact", "lk", "serve"])
+    if op in ("draw", "draw_host", "build"):
+        R = rng.choice([8, 16, 32, 64, 128, rng.randint(2, 16), rng.randint(17, 64), rng.randint(65, 128)])
+        N = rng.randint(2, 6)
+        top = {"draw": 2 ** 27, "draw_host": 2 ** 20, "build": 2 ** 25}[op] // R
+        dims = [_size(rng, 64, top // (1 if N <= 3 else 2)) for _ in range(N)]
+        J = _size(rng, 1024, 2 ** 14 if op == "draw_host" else 2 ** 15 if R > 64 else 2 ** 16)
+        case = {"op": op, "dims": "x".join(map(str, dims)), "R": R, "J": J, "j": rng.choice([N + 1, rng.randrange(N)]),
+                "precision": rng.choice(["fp64", "fp32"]), "factors": rng.choice(["gauss", "graded"])}
+        if op != "draw_host":
+            case["uniforms"] = rng.choice(["given", "builtin"])
+        return case
+    if op == "als":
+        N = rng.choice([3, 3, 4])
+        dims = [_size(rng, 64, 2 ** 19 if N == 3 else 2 ** 12) for _ in range(N)]
+        room = 0.01 * math.prod(float(d) for d in dims)
+        return {"op": "als", "dims": "x".join(map(str, dims)),
+                "nnz": int(min(_size(rng, 5 * 10 ** 5, 10 ** 7), max(room, 2000))),
+                "R": rng.choice([8, 16, 25, rng.randint(9, 32)]), "J": _size(rng, 2 ** 14, 2 ** 16),
+                "host_sync": rng.random() < 0.3}
+    if op == "als_exact":
+        dims = [_size(rng, 512, 2 ** 16) for _ in range(3)]
+        return {"op": "als_exact", "dims": "x".join(map(str, dims)), "nnz": _size(rng, 10 ** 5, 2 * 10 ** 6),
+                "R": rng.choice([8, 16, 25, rng.randint(9, 48)])}
+    if op == "lk":
+        R = rng.choice([8, 16, 32, rng.randint(9, 64)])
+        dims = [_size(rng, 256, 2 ** 24 // R) for _ in range(rng.randint(2, 4))]
+        return {"op": "lk", "dims": "x".join(map(str, dims)), "R": R, "J": _size(rng, 1024, 2 ** 16), "j": len(dims) + 1}
+    return {"op": "serve", "shapes": rng.randrange(1 << 20), "sets": rng.randint(2, 6), "on_sets": rng.randint(4, 24),
+            "fresh": rng.randint(0, 8), "max_log2_rows": rng.randint(14, 19), "precision": rng.choice(["fp32", "fp64"])}
+
+
+def _dims(case):
+    return [int(d) for d in case["dims"].split("x")]
+
+
+# --------------------------------------------------------------------------- inputs
+def _gen(seed):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(int(seed) * 7919 + 17)
+    return g
+
+
+def _factors(dims, R, kind, g):
+    """N(0,1) factors, or ("graded") columns mixed from N(0,1) ones scaled
+    geometrically from 1 to 1e-6."""
+    out = []
+    for n in dims:
+        U = torch.randn((n, R), generator=g, device=DEV, dtype=torch.float64)
+        if kind == "graded":
+            q = np.linalg.qr(torch.randn((R, R), generator=g, device=DEV, dtype=torch.float64).cpu().numpy())[0]
+            mix = np.geomspace(1.0, 1e-6, R)[:, None] * q.T
+            U = U @ torch.from_numpy(np.ascontiguousarray(mix)).to(DEV)
+        out.append(U.contiguous())
+    return out
+
+
+def _zipf(n, size, g):
+    """Zipf(1.1) indices below n by inverse transform of the density x^-1.1."""
+    u = torch.rand(size, generator=g, device=DEV, dtype=torch.float64)
+    x = (1.0 - u * (1.0 - (n + 1.0) ** -0.1)) ** -10.0
+    return (x.floor().to(torch.int64) - 1).clamp_(0, n - 1)
+
+
+def _nonzeros(dims, nnz, g):
+    """At most nnz distinct coordinates, every mode's from a Zipf law, values
+    of a noisy low-rank model: (int64 nnz x N, float64 nnz)."""
+    keys = torch.empty(0, dtype=torch.int64, device=DEV)
+    for _ in range(4):
+        k = torch.zeros(int(1.3 * nnz) + 1000, dtype=torch.int64, device=DEV)
+        for n in dims:
+            k = k * n + _zipf(n, k.numel(), g)
+        keys = torch.unique(torch.cat([keys, k]))
+        if keys.numel() >= nnz:
+            break
+    keys = keys[torch.randperm(keys.numel(), generator=g, device=DEV)[:nnz]]
+    cols = []
+    for n in reversed(dims):
+        cols.append(keys % n)
+        keys = torch.div(keys, n, rounding_mode="floor")
+    idx = torch.stack(cols[::-1], dim=1)
+    vals = torch.zeros(idx.shape[0], dtype=torch.float64, device=DEV)
+    for _ in range(5):
+        p = torch.ones_like(vals)
+        for k, n in enumerate(dims):
+            p *= torch.randn(n, generator=g, device=DEV, dtype=torch.float64)[idx[:, k]]
+        vals += p
+    vals += 0.01 * vals.std() * torch.randn(vals.numel(), generator=g, device=DEV, dtype=torch.float64)
+    return idx, vals
+
+
+def _serve_shapes(case):
+    r = np.random.default_rng(case["shapes"])
+
+    def shape():
+        n = int(r.integers(3, 6))
+        return {"dims": [int(2 ** r.uniform(10, case["max_log2_rows"])) for _ in range(n)],
+                "R": int(r.choice([8, 16, 32, 64])), "J": int(2 ** r.uniform(10, 16))}
+
+    return ([shape() for _ in range(case["sets"])],
+            [(int(r.integers(case["sets"])), int(2 ** r.uniform(10, 16))) for _ in range(case["on_sets"])],
+            [shape() for _ in range(case["fresh"])])
+
+
+class _View:
+    """Device memory at an address, for torch.as_tensor."""
+
+    def __init__(self, ptr, shape):
+        self.__cuda_array_interface__ = {"shape": tuple(shape), "typestr": "<f8", "data": (ptr, False), "version": 3,
+                                         "strides": None}
+
+
+def prepare(case, seed):
+    op, g = case["op"], _gen(seed)
+    s = {"op": op, "case": case}
+    if op in ("draw", "build", "draw_host"):
+        dims, R, J = _dims(case), case["R"], case["J"]
+        N = len(dims)
+        U = _factors(dims, R, case["factors"], g)
+        if op == "draw_host":
+            s["sampler"] = ftl.Sampler([u.cpu().numpy() for u in U], J, R, "efficient", precision=case["precision"])
+            s["sampler"].set_seed(seed, 0)
+            s["out"] = [np.zeros((N, J), dtype=np.uint64), np.zeros((J, R)), np.zeros(J)]
+            return s
+        s["draws"] = (torch.rand(2 * N * J, generator=g, device=DEV, dtype=torch.float64)
+                      if case["uniforms"] == "given" else None)
+        s["out"] = [torch.zeros((N, J), dtype=torch.int64, device=DEV),
+                    torch.zeros((J, R), dtype=torch.float64, device=DEV),
+                    torch.zeros(J, dtype=torch.float64, device=DEV)]
+        s["seed"] = seed
+        if op == "build":
+            s["U"] = U
+        else:
+            s["sampler"] = ftl.Sampler.from_device(U, J, R, case["precision"])
+            s["sampler"].set_seed(seed, 0)
+        return s
+    if op in ("als", "als_exact"):
+        dims, R = _dims(case), case["R"]
+        idx, vals = _nonzeros(dims, case["nnz"], g)
+        U = [u.cpu().numpy() for u in _factors(dims, R, "gauss", g)]
+        s["tensor"] = ftl.SparseTensor.from_device(idx.to(torch.int32).contiguous(), vals, dims=dims)
+        s["model"] = ftl.LowRankTensor(R, U)
+        s["als"] = ftl.ALS(s["model"], s["tensor"], host_sync=case.get("host_sync", False))
+        if op == "als":
+            s["als"].initialize_ds_als(case["J"], seed=seed)
+        s["views"] = [torch.as_tensor(_View(s["als"].factor_device_ptr(k), (n, R)), device=DEV)
+                      for k, n in enumerate(dims)]
+        s["sigma"] = np.zeros(R)
+        return s
+    if op == "lk":
+        dims, R, J = _dims(case), case["R"], case["J"]
+        U = [u.cpu().numpy() for u in _factors(dims, R, "gauss", g)]
+        s["sampler"] = ftl.Sampler(U, J, R, "larsen_kolda")
+        s["draws"] = torch.rand(2 * len(dims) * J, generator=g, device=DEV, dtype=torch.float64)
+        s["out"] = [torch.zeros((len(dims), J), dtype=torch.int64, device=DEV),
+                    torch.zeros((J, R), dtype=torch.float64, device=DEV),
+                    torch.zeros(J, dtype=torch.float64, device=DEV)]
+        return s
+    sets, on_sets, fresh = _serve_shapes(case)
+    s["server"] = ftl.Server(24 << 30, 8)
+    factors = [_factors(q["dims"], q["R"], "gauss", g) for q in sets]
+    torch.cuda.synchronize()  # the server's streams do not follow torch's
+    s["sets"] = [s["server"].add_factors(U, 2 ** 16, case["precision"]) for U in factors]
+    s["on_sets"], s["fresh"], s["seed"] = on_sets, fresh, seed
+    return s
+
+
+# --------------------------------------------------------------------------- one pass
+def run(state):
+    op, case = state["op"], state["case"]
+    if op == "draw_host":
+        state["sampler"].KRPDrawSamples_materialize(case["j"], *state["out"])
+        return state["out"]
+    if op == "draw":
+        state["sampler"].draw_device(case["j"], *state["out"], state["draws"])
+        return state["out"]
+    if op == "build":
+        sampler = ftl.Sampler.from_device(state["U"], case["J"], case["R"], case["precision"])
+        sampler.set_seed(state["seed"], 0)
+        sampler.draw_device(case["j"], *state["out"], state["draws"])
+        sampler.close()
+        return state["out"]
+    if op == "als":
+        for j in range(state["model"].N):
+            state["als"].execute_ds_als_update(j, True, True)
+        state["model"].get_sigma(state["sigma"])
+        return (state["model"].U if case["host_sync"] else state["views"]) + [state["sigma"]]
+    if op == "als_exact":
+        for j in range(state["model"].N):
+            state["als"].execute_exact_als_update(j, True, True)
+        state["model"].get_sigma(state["sigma"])
+        return state["views"] + [state["sigma"], state["als"].residual_normsq()]
+    if op == "lk":
+        state["sampler"].update_sampler(0)
+        state["sampler"].draw_device(case["j"], *state["out"], state["draws"])
+        return state["out"]
+    srv, seed = state["server"], state["seed"]
+    ids = [srv.submit_on(state["sets"][k], J, None, seed + i) for i, (k, J) in enumerate(state["on_sets"])]
+    ids += [srv.submit(q["dims"], q["R"], q["J"], None, seed + 1000 + i, case["precision"])
+            for i, q in enumerate(state["fresh"])]
+    return [srv.wait(i) for i in ids]
+
+
+# --------------------------------------------------------------------------- floors
+def _draw_work(dims, R, J, j, precision):
+    """Every node and leaf block that J samples reach read once, in the storage
+    of the sampler's precision, and the outputs written once."""
+    T, b, f = R * (R + 1) // 2, 0.0, 0.0
+    for k, n in enumerate(dims):
+        if k == j:
+            continue
+        leaves = max(1, -(-n // min(n, R)))
+        levels = int(math.ceil(math.log2(leaves)))
+        for d in range(levels + 1):
+            nodes = max(1.0, 2.0 ** d / 2)
+            seen = -nodes * math.expm1(J * math.log1p(-1.0 / nodes)) if nodes > 1 else 1.0
+            b += seen * T * (4 if precision == "fp32" and d > levels - 4 else 8)
+        seen = -leaves * math.expm1(J * math.log1p(-1.0 / leaves)) if leaves > 1 else 1.0
+        b += seen * min(n, R) * R * (4 if precision == "fp32" else 8) + J * 8
+        f += J * (2.0 * T * (levels + 2 + math.log2(R)) + 2.0 * R * R)
+    return b + J * (R + 1) * 8, f + 2.0 * J * R * R
+
+
+def _build_work(dims, R, precision):
+    T, b, f = R * (R + 1) // 2, 0.0, 0.0
+    for n in dims:
+        leaves = -(-n // min(n, R))
+        b += n * R * 8 + 2 * leaves * T * (4 if precision == "fp32" else 8) + (n * R * 4 if precision == "fp32" else 0)
+        f += 2.0 * n * T + leaves * T
+    return b, f
+
+
+def work(case):
+    op = case["op"]
+    if op in ("draw", "draw_host", "build"):
+        b, f = _draw_work(_dims(case), case["R"], case["J"], case["j"], case["precision"])
+        if op == "build":
+            b2, f2 = _build_work(_dims(case), case["R"], case["precision"])
+            b, f = b + b2, f + f2
+        return {"bytes": b, "flops": f}
+    if op == "als":
+        b = f = 0.0
+        dims, R, J = _dims(case), case["R"], case["J"]
+        for j, n in enumerate(dims):
+            bd, fd = _draw_work(dims, R, J, j, "fp64")
+            bb, fb = _build_work([n], R, "fp64")
+            b += bd + bb + n * R * 8 + J * R * 8
+            f += fd + fb + J * R * (R + 1) + 2.0 * n * R * R
+        return {"bytes": b, "flops": f}
+    if op == "als_exact":
+        dims, R, nnz = _dims(case), case["R"], case["nnz"]
+        N = len(dims)
+        per = nnz * (8 + 4 * N) + sum(dims) * R * 8
+        return {"bytes": float((N + 1) * per), "flops": float((N + 1) * nnz * R * (N + 1) + 2 * sum(dims) * R * R * N)}
+    if op == "lk":
+        dims, R, J = _dims(case), case["R"], case["J"]
+        return {"bytes": float(dims[0] * R * 8 + dims[0] * 8 + J * (len(dims) * (R + 2) + R + 1) * 8),
+                "flops": float(dims[0] * (R * R + 2 * R * R) + J * len(dims) * R)}
+    sets, on_sets, fresh = _serve_shapes(case)
+    b = f = 0.0
+    for q, J in [(sets[k], J) for k, J in on_sets] + [(q, q["J"]) for q in fresh]:
+        bd, fd = _draw_work(q["dims"], q["R"], J, -1, case["precision"])
+        b, f = b + bd, f + fd
+    for q in fresh:
+        bb, fb = _build_work(q["dims"], q["R"], case["precision"])
+        b, f = b + bb + sum(q["dims"]) * q["R"] * 8, f + fb
+    return {"bytes": b, "flops": f}
+
+
+# --------------------------------------------------------------------------- 64-bit results
+def _philox(seed, call, J, stage):
+    """Uniforms of the built-in generator: Philox4x32-10 at counter (sample,
+    stage, call), 53 bits of the first two words."""
+    mask = np.uint64(0xFFFFFFFF)
+    i = np.arange(J, dtype=np.uint64)
+    c = [i & mask, (i >> np.uint64(32)) ^ np.uint64(stage << 16), np.full(J, call & 0xFFFFFFFF, np.uint64),
+         np.full(J, call >> 32, np.uint64)]
+    k = [seed & 0xFFFFFFFF, seed >> 32]
+    for _ in range(10):
+        p0, p1 = np.uint64(0xD2511F53) * c[0], np.uint64(0xCD9E8D57) * c[2]
+        c = [(p1 >> np.uint64(32)) ^ c[1] ^ np.uint64(k[0]), p1 & mask,
+             (p0 >> np.uint64(32)) ^ c[3] ^ np.uint64(k[1]), p0 & mask]
+        k = [(k[0] + 0x9E3779B9) & 0xFFFFFFFF, (k[1] + 0xBB67AE85) & 0xFFFFFFFF]
+    v = (c[0] >> np.uint64(5)) * np.uint64(1 << 26) + (c[1] >> np.uint64(6))
+    return v.astype(np.float64) / 2.0 ** 53
+
+
+def _uniforms(seed, call, N, J):
+    d = [_philox(seed, call, J, 2 * k) for k in range(N)] + [_philox(seed, call, J, 2 * k + 1) for k in range(N)]
+    return torch.from_numpy(np.concatenate(d)).to(DEV)
+
+
+def _eigh(G):
+    lam, V = np.linalg.eigh(G.cpu().numpy())
+    return torch.from_numpy(lam).to(DEV), torch.from_numpy(V).to(DEV)
+
+
+def _pick_rows(U, X, u):
+    """First row of U at which the running sum of (row . x)^2 reaches u of its
+    total, for each x (rows of X)."""
+    B, n = 1024, U.shape[0]
+    pad = (-n) % B
+    if pad:
+        U = torch.cat([U, U.new_zeros((pad, U.shape[1]))])
+    out, step = [], max(1, 2 ** 28 // U.shape[0])
+    for a in range(0, X.shape[0], step):
+        x = X[a:a + step]
+        P = (x @ U.T).square_().view(x.shape[0], -1, B)
+        S = P.sum(2)
+        C = S.cumsum(1)
+        t = (u[a:a + step] * C[:, -1])[:, None].contiguous()
+        b = torch.searchsorted(C, t).clamp_(max=S.shape[1] - 1)
+        base = C.gather(1, b) - S.gather(1, b)
+        rows = P.gather(1, b[:, :, None].expand(-1, 1, B))[:, 0].cumsum(1) + base
+        r = torch.searchsorted(rows, t).clamp_(max=B - 1)
+        out.append((b * B + r)[:, 0].clamp_(max=n - 1))
+    return torch.cat(out)
+
+
+def _exact_draw(U, J, j, draws):
+    """(samples, h, weights) of the leverage draw by brute force."""
+    N, R = len(U), U[0].shape[1]
+    modes = [k for k in range(N) if k != j]
+    G = {k: U[k].T @ U[k] for k in modes}
+    full = torch.ones((R, R), dtype=torch.float64, device=DEV)
+    for k in modes:
+        full = full * G[k]
+    lam, V = _eigh(full)
+    keep = (lam > 1e-8).to(lam)
+    W = V * (keep / torch.where(lam > 1e-8, lam, torch.ones_like(lam)).sqrt())
+    pinv = W @ W.T
+    h = torch.ones((J, R), dtype=torch.float64, device=DEV)
+    samples = torch.zeros((N, J), dtype=torch.int64, device=DEV)
+    for t, k in enumerate(modes):
+        if t + 1 < len(modes):
+            P = pinv.clone()
+            for q in modes[t + 1:]:
+                P = P * G[q]
+            mu, Q = _eigh(P)
+            E = (Q * mu.clamp(min=0).sqrt()).T
+        else:
+            E = W.flip(1).T
+        mass = torch.stack([((h * e) @ G[k] * (h * e)).sum(1) for e in E], dim=1).cumsum(1)
+        ue, ug = draws[k * J:(k + 1) * J], draws[(N + k) * J:(N + k + 1) * J]
+        r = torch.searchsorted(mass, (ue * mass[:, -1])[:, None].contiguous()).clamp_(max=R - 1)[:, 0]
+        samples[k] = _pick_rows(U[k], h * E[r], ug)
+        h = h * U[k][samples[k]]
+    return samples, h, R / (J * ((h @ pinv) * h).sum(1))
+
+
+def _solve(M, A, R):
+    lam, V = _eigh(A)
+    keep = lam > 1e-11
+    W = V[:, keep]
+    out = M @ ((W / lam[keep]) @ W.T)
+    norm = out.square().sum(0).sqrt()
+    norm = torch.where(norm < 1e-7, torch.ones_like(norm), norm)
+    return out / norm, norm
+
+
+def _exact_als(case, seed):
+    dims, R = _dims(case), case["R"]
+    N, g = len(dims), _gen(seed)
+    idx, vals = _nonzeros(dims, case["nnz"], g)
+    U = _factors(dims, R, "gauss", g)
+    sigma = torch.ones(R, dtype=torch.float64, device=DEV)
+    for j in range(N):
+        M = torch.zeros((dims[j], R), dtype=torch.float64, device=DEV)
+        if case["op"] == "als":
+            J = case["J"]
+            samples, h, w = _exact_draw(U, J, j, _uniforms(seed, j, N, J))
+            key = torch.zeros(J, dtype=torch.int64, device=DEV)
+            nz = torch.zeros(idx.shape[0], dtype=torch.int64, device=DEV)
+            for k in range(N):
+                if k != j:
+                    key, nz = key * dims[k] + samples[k], nz * dims[k] + idx[:, k]
+            uniq, inv, count = torch.unique(key, return_inverse=True, return_counts=True)
+            first = torch.full_like(uniq, J).scatter_reduce_(0, inv, torch.arange(J, device=DEV), "amin")
+            hu, wu = h[first], (w[first] * count)[:, None]
+            A = (hu * wu).T @ hu
+            at = torch.searchsorted(uniq, nz).clamp_(max=uniq.numel() - 1)
+            hit = (uniq[at] == nz).nonzero()[:, 0]
+            for part in hit.split(1 << 22):
+                M.index_add_(0, idx[part, j], vals[part, None] * (hu * wu)[at[part]])
+        else:
+            A = torch.ones((R, R), dtype=torch.float64, device=DEV)
+            for k in range(N):
+                if k != j:
+                    A = A * (U[k].T @ U[k])
+            for z in torch.arange(idx.shape[0], device=DEV).split(1 << 22):
+                p = vals[z, None].expand(-1, R)
+                for k in range(N):
+                    if k != j:
+                        p = p * U[k][idx[z, k]]
+                M.index_add_(0, idx[z, j], p)
+        U[j], sigma = _solve(M, A, R)
+    return U, sigma, idx, vals
+
+
+def exact(case, seed):
+    op = case["op"]
+    if op == "serve":
+        return None
+    dims, R = _dims(case), case["R"]
+    N, J = len(dims), case.get("J", 0)
+    if op in ("draw", "draw_host", "build"):
+        if J * sum(n for k, n in enumerate(dims) if k != case["j"]) > BRUTE_LIMIT:
+            return None
+        g = _gen(seed)
+        U = _factors(dims, R, case["factors"], g)
+        if case.get("uniforms") == "given":
+            draws = torch.rand(2 * N * J, generator=g, device=DEV, dtype=torch.float64)
+        else:
+            draws = _uniforms(seed, 0, N, J)
+        samples, h, w = _exact_draw(U, J, case["j"], draws)
+        return [None, h.cpu().numpy(), w.cpu().numpy()] if op == "draw_host" else [None, h, w]
+    if op == "lk":
+        g = _gen(seed)
+        U = _factors(dims, R, "gauss", g)
+        draws = torch.rand(2 * N * J, generator=g, device=DEV, dtype=torch.float64)
+        h, p = torch.ones((J, R), dtype=torch.float64, device=DEV), torch.ones(J, dtype=torch.float64, device=DEV)
+        for k in range(N):
+            lev = ((U[k] @ torch.linalg.inv(U[k].T @ U[k])) * U[k]).sum(1)
+            C = lev.cumsum(0)
+            r = torch.searchsorted(C, draws[k * J:(k + 1) * J] * C[-1], right=True).clamp_(max=dims[k] - 1)
+            h, p = h * U[k][r], p * (lev[r] / C[-1])
+        return [None, h, 1.0 / (J * p)]
+    if op == "als" and J * sum(dims) * (N - 1) > BRUTE_LIMIT:
+        return None
+    try:
+        U, sigma, idx, vals = _exact_als(case, seed)
+    except np.linalg.LinAlgError:  # too few matches: a factor of zeros, then NaN
+        return None
+    if op == "als":
+        return [u.cpu().numpy() if case["host_sync"] else u for u in U] + [sigma.cpu().numpy()]
+    inner = torch.zeros((), dtype=torch.float64, device=DEV)
+    for z in torch.arange(idx.shape[0], device=DEV).split(1 << 22):
+        p = sigma.expand(z.numel(), -1)
+        for k in range(N):
+            p = p * U[k][idx[z, k]]
+        inner += (p.sum(1) * vals[z]).sum()
+    A = sigma[:, None] * sigma[None, :]
+    for k in range(N):
+        A = A * (U[k].T @ U[k])
+    return U + [sigma.cpu().numpy(), float(vals.square().sum() - 2 * inner + A.sum())]
