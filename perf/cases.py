@@ -171,9 +171,11 @@ def _serve_shapes(case):
 
 
 class _View:
-    """Device memory at an address, for torch.as_tensor."""
+    """Device memory at an address, for torch.as_tensor, which keeps this object
+    and so the memory's owner alive as long as the tensor."""
 
-    def __init__(self, ptr, shape):
+    def __init__(self, owner, ptr, shape):
+        self.owner = owner
         self.__cuda_array_interface__ = {"shape": tuple(shape), "typestr": "<f8", "data": (ptr, False), "version": 3,
                                          "strides": None}
 
@@ -211,7 +213,7 @@ def prepare(case, seed):
         s["als"] = ftl.ALS(s["model"], s["tensor"], host_sync=case.get("host_sync", False))
         if op == "als":
             s["als"].initialize_ds_als(case["J"], seed=seed)
-        s["views"] = [torch.as_tensor(_View(s["als"].factor_device_ptr(k), (n, R)), device=DEV)
+        s["views"] = [torch.as_tensor(_View(s["als"], s["als"].factor_device_ptr(k), (n, R)), device=DEV)
                       for k, n in enumerate(dims)]
         s["sigma"] = np.zeros(R)
         return s
