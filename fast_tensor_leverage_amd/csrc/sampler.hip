@@ -357,6 +357,12 @@ inline unsigned grid_for(uint64_t work, unsigned bs) {
 
 }  // namespace
 
+// Largest J whose samples are ordered (kOrderMaxBlocks sort blocks of at most
+// 65,536 samples).
+constexpr uint64_t kOrderMaxJ = 1ull << 24;
+
+inline uint64_t order_blocks(uint64_t J) { return (J + order_share(J) - 1) / order_share(J); }
+
 struct Sampler {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -428,14 +434,11 @@ struct Sampler {
     uint32_t draw_kernel = 0;
     // threads per block of the one-sample-per-block kernel (0: by rank)
     uint32_t block_threads = 0;
-    // 1: each mode's descent bucketed by level-3 subtree onto XCD-affine
-    // blocks.  Measured at N=3, I=2^23, R=32 (FP64): prefix 167 + partition
-    // 97 + suffix 367 us per mode against 539 us for the one-launch mode, so
-    // off by default: the per-level cost does not depend on where the node
-    // is cached.
-    uint32_t xcd_buckets = 0;
-    double *st_x = nullptr, *st_s = nullptr;
-    uint32_t *bucket = nullptr, *blist = nullptr, *boff = nullptr;
+    // option "sample_order": launches take the samples by increasing Gram
+    // uniform (0 never, 1 always, 2 by order_pays)
+    uint32_t sample_order = 2;
+    uint16_t* order_bin = nullptr;
+    uint32_t *order_count = nullptr, *order_perm = nullptr;
     double* h_state = nullptr;
     bool timing = false;
     // events of every timed call since the last read-out: {start, after
@@ -748,9 +751,12 @@ struct Sampler {
         } else if (key == "grid_blocks") {
             FTL_REQUIRE(value >= 0, "grid_blocks must be >= 0");
             grid_override = (uint32_t)value;
+        } else if (key == "sample_order") {
+            FTL_REQUIRE(value >= 0 && value <= 2, "sample_order must be 0, 1 or 2");
+            sample_order = (uint32_t)value;
         } else if (key == "xcd_buckets") {
             FTL_REQUIRE(value == 0 || value == 1, "xcd_buckets must be 0 or 1");
-            xcd_buckets = (uint32_t)value;
+            sample_order = value ? 1 : 2;
         } else if (key == "draw_kernel") {
             FTL_REQUIRE(value >= 0 && value <= 3, "draw_kernel must be 0, 1, 2 or 3");
             draw_kernel = (uint32_t)value;
@@ -826,7 +832,8 @@ struct Sampler {
         if (key == "draw_kernel") return draw_kernel;
         if (key == "block_threads") return block_threads;
         if (key == "overlap_compute_m") return overlap_cm && n_msets > 1;
-        if (key == "xcd_buckets") return xcd_buckets;
+        if (key == "sample_order") return sample_order;
+        if (key == "xcd_buckets") return sample_order == 1;
         if (key == "jacobi_threads") return jacobi_override ? jacobi_override : jacobi_threads_for(R);
         if (key == "fp32_levels") return fp32_levels;
         if (key == "fp32_leaf") return leaf32;
@@ -956,11 +963,11 @@ struct Sampler {
         work = msets[0].work;
         lam = msets[0].lam;
         h_state = dalloc<double>(J * R);
-        st_x = dalloc<double>(J * R);
-        st_s = dalloc<double>(J * 4);
-        bucket = dalloc<uint32_t>(J);
-        blist = dalloc<uint32_t>(J);
-        boff = dalloc<uint32_t>(kBuckets + 1);
+        if (J <= kOrderMaxJ) {
+            order_bin = dalloc<uint16_t>(N * J);
+            order_perm = dalloc<uint32_t>(N * J);
+            order_count = dalloc<uint32_t>(N * order_blocks(J) * kOrderBins);
+        }
         trees_dirty = true;
         if (sync_end) FTL_HIP_CHECK(hipStreamSynchronize(stream));
     }
@@ -996,7 +1003,8 @@ struct Sampler {
         const uint64_t R2 = R * R;
         total += up(R2 * 8) * 2 + up(N * R2 * 8) + up(((uint64_t)N * (2 * R - 1) * ts64 + pad) * 8) +
                  up((uint64_t)(N + 1) * 3 * (R + 1) * R * 8) + up((uint64_t)(N + 1) * R * 8);
-        total += up(J * R * 8) * 2 + up(J * 4 * 8) + up(J * 4) * 2 + up((kBuckets + 1) * 4);
+        total += up(J * R * 8);
+        if (J <= kOrderMaxJ) total += up(N * J * 2) + up(N * J * 4) + up(N * order_blocks(J) * kOrderBins * 4);
         return total;
     }
 
@@ -1175,27 +1183,41 @@ struct Sampler {
         with_cfg([&](auto rmax, auto sgc) { launch_draw_p<decltype(rmax)::value, decltype(sgc)::value>(a, st); });
     }
 
-    // The bucketed draw of sampled mode a.mi_begin: prefix, partition, suffix.
-    void dispatch_bucketed(const DrawArgs& a, hipStream_t st) {
-        with_cfg([&](auto rmax, auto sgc) {
-            constexpr int RM = decltype(rmax)::value, SG = decltype(sgc)::value, BS = 256;
-            const uint64_t per_block = BS / SG;
-            const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>((J + per_block - 1) / per_block, 1u << 20));
-            hipLaunchKernelGGL((k_draw_prefix<RM, SG, BS>), dim3((unsigned)blocks), dim3(BS), 0, st, a);
-            FTL_HIP_CHECK(hipGetLastError());
-            hipLaunchKernelGGL(k_bucket_partition<1024>, dim3(1), dim3(1024), 0, st, a.bucket, J, a.blist, a.boff);
-            FTL_HIP_CHECK(hipGetLastError());
-            // kBuckets x the blocks one bucket of J / kBuckets samples needs
-            const uint64_t per_bucket = (J + kBuckets - 1) / kBuckets;
-            const uint64_t sblocks = kBuckets * std::max<uint64_t>(1, (per_bucket + per_block - 1) / per_block);
-            if (precision == FTL_FP32)
-                hipLaunchKernelGGL((k_draw_suffix<RM, SG, BS, true>), dim3((unsigned)std::min<uint64_t>(sblocks, 1u << 20)),
-                                   dim3(BS), 0, st, a);
-            else
-                hipLaunchKernelGGL((k_draw_suffix<RM, SG, BS, false>), dim3((unsigned)std::min<uint64_t>(sblocks, 1u << 20)),
-                                   dim3(BS), 0, st, a);
-            FTL_HIP_CHECK(hipGetLastError());
-        });
+    // When the order is made: nodes of 1.1 KB or more (R > 16), some tree of
+    // 16 MB, four times an XCD's L2, and samples enough to share its nodes.
+    // Draw kernels of a call, in order against 0..J-1: I = 2^23, R = 32, J =
+    // 50,000 FP32 836 / 977 us; I = 2^22 FP64 (two modes) 600 / 742; I = 2^20,
+    // R = 128 FP32 13.8 / 16.8 ms, R = 64 2.6 / 3.2 ms; I = 2^18, R = 32, J =
+    // 8192 149 / 175 us, J = 2048 67 / 72.  Smaller trees and nodes gain less
+    // than the sort (15 us beside computeM) and the indirection may cost: I =
+    // 2^14, R = 32 511 / 530; I = 2^18, R = 16, six modes 453 / 475, but 578 /
+    // 570 a call when samplers alternate; I = 1000, R = 8 47 / 45.
+    bool order_pays() const {
+        if (J < 2048 || R <= 16) return false;
+        for (const ModeHost& m : modes)
+            if (m.sh.node_count * ts64 * sizeof(double) >= (16u << 20)) return true;
+        return false;
+    }
+    bool ordered() const { return order_perm && (sample_order == 1 || (sample_order == 2 && order_pays())); }
+
+    // The order of every sampled mode's samples (k_order_*), queued on st.
+    void make_order(const std::vector<int>& order, const double* draws, hipStream_t st) {
+        OrderArgs o{};
+        for (size_t t = 0; t < order.size(); t++) o.modes[t] = order[t];
+        o.N = (int)N;
+        o.J = J;
+        o.draws = draws;
+        o.seed = seed;
+        o.call = call;
+        o.share = order_share(J);
+        o.bin = order_bin;
+        o.count = order_count;
+        o.perm = order_perm;
+        const dim3 grid((unsigned)order_blocks(J), (unsigned)order.size());
+        hipLaunchKernelGGL(k_order_count, grid, dim3(256), 0, st, o);
+        FTL_HIP_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(k_order_scatter, grid, dim3(256), 0, st, o);
+        FTL_HIP_CHECK(hipGetLastError());
     }
 
     // Kernel arguments of one draw over the sampled modes `order` reading the
@@ -1234,12 +1256,6 @@ struct Sampler {
         a.samples = samples;
         a.h_out = h;
         a.w_out = w;
-        a.split_level = kBucketLevel;
-        a.st_x = st_x;
-        a.st_s = st_s;
-        a.bucket = bucket;
-        a.blist = blist;
-        a.boff = boff;
         a.mi_begin = 0;
         a.mi_end = a.m;
         a.h_state = nullptr;
@@ -1262,6 +1278,7 @@ struct Sampler {
         if (timing)
             for (auto& e : evs) e = take_event();
         const bool overlap = overlap_cm && n_msets > 1;
+        const bool by_order = ordered();
         const MSet& ms = msets[overlap ? (mset_next++ & 1) : 0];
         if (overlap) {
             if (trees_dirty) {
@@ -1272,8 +1289,10 @@ struct Sampler {
             FTL_HIP_CHECK(hipStreamWaitEvent(cm_stream, ms.draw_done, 0));
             compute_m(j, cm_stream, ms, timing ? evs.data() : nullptr);
             FTL_HIP_CHECK(hipEventRecord(ms.cm_done, cm_stream));
+            if (by_order) make_order(order, draws, st);
             FTL_HIP_CHECK(hipStreamWaitEvent(st, ms.cm_done, 0));
         } else {
+            if (by_order) make_order(order, draws, st);
             compute_m(j, st, ms, timing ? evs.data() : nullptr);
         }
         if (timing) FTL_HIP_CHECK(hipEventRecord(evs[3], st));
@@ -1283,15 +1302,14 @@ struct Sampler {
             for (int mi = 0; mi < a.m; mi++) {
                 a.mi_begin = mi;
                 a.mi_end = mi + 1;
-                // bucketed when the tree is deep enough for the split to matter
-                if (xcd_buckets && draw_kernel == 0 && R <= 64 && modes[a.order[mi]].sh.lfill_level >= 8)
-                    dispatch_bucketed(a, st);
-                else dispatch_draw(a, st);
+                a.perm = by_order ? order_perm + (uint64_t)mi * J : nullptr;
+                dispatch_draw(a, st);
             }
         } else {
             a.mi_begin = 0;
             a.mi_end = a.m;
             a.h_state = nullptr;
+            a.perm = by_order ? order_perm : nullptr;
             dispatch_draw(a, st);
         }
         if (overlap) FTL_HIP_CHECK(hipEventRecord(ms.draw_done, st));

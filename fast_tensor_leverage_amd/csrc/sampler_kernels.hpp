@@ -7,6 +7,7 @@
 //                   eigendecomposition and pinv (efficient_krp_sampler.hpp:90-150)
 //   k_eigen_modes   computeM part 2: per-mode eigen matrices E_k and eigen
 //                   trees (efficient_krp_sampler.hpp:152-193)
+//   k_order_*       the order in which a mode's launch takes the samples
 //   k_krp_draw      the whole KRPDrawSamples after computeM, fused: for every
 //                   sample, every sampled mode's eigen descent, Gram descent,
 //                   leaf row scan and h update, then the weight
@@ -833,24 +834,124 @@ struct DrawArgs {
     // FP32 samplers: leaf scans over the FP32 factor copy (1) or the FP64
     // factors (0)
     int leaf32;
-    // subtree-bucketed descent of one mode (k_draw_prefix / k_draw_suffix):
-    // per-sample x (J x R) and {low, high, m, node} (J x 4) after the first
-    // split_level levels, the level-split_level subtree of each sample and
-    // the samples grouped by subtree (offsets: kBuckets + 1 entries)
-    uint32_t split_level;
-    double* st_x;
-    double* st_s;
-    uint32_t* bucket;
-    uint32_t* blist;
-    uint32_t* boff;
+    // the order in which the launch goes through the samples (J indices, by
+    // k_order_*), or null for 0..J-1
+    const uint32_t* perm;
 };
 
-// Subtrees of the bucketed descent: one per XCD (8 on MI355X).  Workgroups
-// are dispatched to the XCDs round-robin, so block b runs on XCD b % 8 and
-// the suffix kernel gives bucket b % 8 to block b: each XCD's L2 then holds
-// the nodes of one subtree only, eight times fewer than the whole tree.
-constexpr uint32_t kBuckets = 8;
-constexpr uint32_t kBucketLevel = 3;
+// ---------------------------------------------------------------------------
+// Order of the samples in a mode's launch.  A descent's leaf is near the
+// u-quantile of the rows, so samples taken by increasing Gram uniform reach
+// neighbouring subtrees one after the other: waves that run at the same time
+// then read the same nodes, and the order is cut into one contiguous part per
+// XCD (ordered_block), so that each L2 sees an eighth of the tree and fetches a
+// node once instead of once per XCD and eviction.  A sample's result does not
+// depend on its place, so only a counting sort by the uniform's leading bits
+// is needed (the order inside a bin is arbitrary), for every sampled mode of
+// the call at once, beside computeM.  Blocks of the sort count their share of
+// the samples in LDS and write the counts out; the second kernel's blocks each
+// sum the table up to their own entries (device-scope atomics on one table
+// took 34 us for three modes of 50,000 samples, most of it their round trips).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kOrderBins = 2048;
+constexpr uint32_t kOrderMaxBlocks = 256;
+constexpr uint32_t kXcds = 8;
+
+// Samples per sort block (a multiple of its 256 threads).
+__host__ __device__ inline uint32_t order_share(uint64_t J) {
+    const uint64_t s = (J + kOrderMaxBlocks - 1) / kOrderMaxBlocks;
+    return s <= 2048 ? 2048u : (uint32_t)((s + 255) / 256 * 256);
+}
+
+struct OrderArgs {
+    int modes[kMaxModes];  // sampled modes; blockIdx.y is the position
+    int N;
+    uint64_t J;
+    uint32_t share;        // order_share(J); gridDim.x = ceil(J / share)
+    const double* draws;   // 2*N*J or null (Philox)
+    uint64_t seed, call;
+    uint16_t* bin;         // m x J
+    uint32_t* count;       // m x gridDim.x x kOrderBins
+    uint32_t* perm;        // m x J
+};
+
+__global__ void __launch_bounds__(256) k_order_count(OrderArgs a) {
+    __shared__ uint32_t cnt[kOrderBins];
+    for (uint32_t b = threadIdx.x; b < kOrderBins; b += 256) cnt[b] = 0;
+    __syncthreads();
+    const uint32_t t = blockIdx.y;
+    const int k = a.modes[t];
+    const uint64_t i0 = (uint64_t)blockIdx.x * a.share, i1 = min(i0 + a.share, a.J);
+    const double* u_given = a.draws ? a.draws + ((uint64_t)a.N + k) * a.J : nullptr;
+#pragma unroll 8
+    for (uint64_t i = i0 + threadIdx.x; i < i1; i += 256) {
+        const double u = u_given ? u_given[i] : philox_uniform(a.seed, a.call, i, 2 * k + 1);
+        const uint32_t b = u >= 1.0 ? kOrderBins - 1 : u > 0.0 ? (uint32_t)(u * kOrderBins) : 0u;
+        a.bin[t * a.J + i] = (uint16_t)b;
+        atomicAdd(cnt + b, 1u);
+    }
+    __syncthreads();
+    uint32_t* out = a.count + ((uint64_t)t * gridDim.x + blockIdx.x) * kOrderBins;
+    for (uint32_t b = threadIdx.x; b < kOrderBins; b += 256) out[b] = cnt[b];
+}
+
+__global__ void __launch_bounds__(256) k_order_scatter(OrderArgs a) {
+    constexpr int PT = kOrderBins / 256;
+    __shared__ uint32_t at[kOrderBins];
+    __shared__ uint32_t wsum[4];
+    const uint32_t t = blockIdx.y;
+    // bins PT * threadIdx.x + q: their samples in all blocks, and in the
+    // blocks before this one
+    uint32_t all[PT], before[PT];
+#pragma unroll
+    for (int q = 0; q < PT; q++) all[q] = before[q] = 0;
+    const uint32_t* src = a.count + (uint64_t)t * gridDim.x * kOrderBins + threadIdx.x * PT;
+#pragma unroll 4
+    for (uint32_t b = 0; b < gridDim.x; b++) {
+        const uint4 c0 = *reinterpret_cast<const uint4*>(src + b * kOrderBins);
+        const uint4 c1 = *reinterpret_cast<const uint4*>(src + b * kOrderBins + 4);
+        const uint32_t c[PT] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        const uint32_t own = b < blockIdx.x ? ~0u : 0u;
+#pragma unroll
+        for (int q = 0; q < PT; q++) {
+            all[q] += c[q];
+            before[q] += c[q] & own;
+        }
+    }
+    uint32_t run = 0;
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+        before[q] += run;
+        run += all[q];
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t incl = run;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    uint32_t base = incl - run;
+    for (int q = 0; q < w; q++) base += wsum[q];
+#pragma unroll
+    for (int q = 0; q < PT; q++) at[threadIdx.x * PT + q] = base + before[q];
+    __syncthreads();
+    const uint64_t i0 = (uint64_t)blockIdx.x * a.share, i1 = min(i0 + a.share, a.J);
+#pragma unroll 8
+    for (uint64_t i = i0 + threadIdx.x; i < i1; i += 256) {
+        const uint32_t pos = atomicAdd(at + a.bin[t * a.J + i], 1u);
+        a.perm[t * a.J + pos] = (uint32_t)i;
+    }
+}
+
+// Blocks go to the XCDs round-robin: block b of n takes place ordered_block(b, n),
+// a bijection of [0, n) that gives each XCD one contiguous range.
+__device__ inline uint32_t ordered_block(uint32_t b, uint32_t n) {
+    const uint32_t x = b % kXcds, q = n / kXcds, r = n % kXcds;
+    return x * q + min(x, r) + b / kXcds;
+}
 
 template <int RMAX, int SG>
 struct DrawCfg {
@@ -1142,8 +1243,9 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
     const int R = a.R;
     const int T = (int)tri_size(R);
     constexpr bool fp32 = USE32;
-    const uint64_t i = item * GPW + lane / SG;
-    const bool active = i < a.J;
+    const uint64_t slot = item * GPW + lane / SG;
+    const bool active = slot < a.J;
+    const uint64_t i = active && a.perm ? a.perm[slot] : slot;
     double h[HPL];
 #pragma unroll
     for (int k = 0; k < HPL; k++) h[k] = 1.0;
@@ -1251,7 +1353,8 @@ __global__ void __launch_bounds__(BS) k_krp_draw(DrawArgs a) {
     for (int b = g; b < RMAX; b += SG) xs[b] = 0.0;
     wave_sync_lds();
     const uint64_t waves_total = (uint64_t)gridDim.x * (BS / 64);
-    const uint64_t wave_id = (uint64_t)blockIdx.x * (BS / 64) + wave;
+    const uint32_t block = a.perm ? ordered_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint64_t wave_id = (uint64_t)block * (BS / 64) + wave;
     const uint64_t n_items = (a.J + GPW - 1) / GPW;
     for (uint64_t item = wave_id; item < n_items; item += waves_total)
         krp_draw_item<RMAX, SG, USE32>(a, item, xs, qs, pair_tab, lane, g);
@@ -1371,7 +1474,9 @@ __global__ void __launch_bounds__(BS) k_krp_draw_wave(DrawArgs a) {
     for (int b = lane; b < RMAX; b += 64) xs[b] = 0.0;
     wave_sync_lds();
     const uint64_t waves_total = (uint64_t)gridDim.x * WPB;
-    for (uint64_t i = (uint64_t)blockIdx.x * WPB + wave; i < a.J; i += waves_total) {
+    const uint32_t block = a.perm ? ordered_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    for (uint64_t slot = (uint64_t)block * WPB + wave; slot < a.J; slot += waves_total) {
+        const uint64_t i = a.perm ? a.perm[slot] : slot;
         double h[HPL];
 #pragma unroll
         for (int q = 0; q < HPL; q++) h[q] = 1.0;
@@ -1646,7 +1751,17 @@ __global__ void __launch_bounds__(BS) k_krp_draw_block(DrawArgs a) {
     for (int b = tid; b < RMAX; b += BS) xs[b] = 0.0;
     __syncthreads();
 
-    for (uint64_t i = blockIdx.x; i < a.J; i += gridDim.x) {
+    // Ordered: the blocks of XCD x = blockIdx % 8 share the x-th eighth of the
+    // order, neighbouring samples at the same time.
+    uint64_t first = blockIdx.x, end = a.J, step = gridDim.x;
+    if (a.perm && gridDim.x >= kXcds) {
+        const uint32_t x = blockIdx.x % kXcds;
+        first = a.J * x / kXcds + blockIdx.x / kXcds;
+        end = a.J * (x + 1) / kXcds;
+        step = gridDim.x / kXcds + (x < gridDim.x % kXcds ? 1 : 0);
+    }
+    for (uint64_t slot = first; slot < end; slot += step) {
+        const uint64_t i = a.perm ? a.perm[slot] : slot;
         double h = 1.0;  // thread tid < R owns h[tid]
         if (a.mi_begin > 0 && tid < R) h = a.h_state[i * R + tid];
         for (int mi = a.mi_begin; mi < a.mi_end; mi++) {
@@ -1711,235 +1826,6 @@ __global__ void __launch_bounds__(BS) k_krp_draw_block(DrawArgs a) {
         if (tid == 0 && a.w_out) a.w_out[i] = (double)R / (lev * (double)a.J);
         if (a.h_out && tid < R) a.h_out[i * R + tid] = h;
         __syncthreads();
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Subtree-bucketed draw of one sampled mode (positions mi_begin, one launch
-// each): k_draw_prefix runs the eigen stage and the first split_level Gram
-// levels and records the state, k_bucket_partition groups the samples by
-// their subtree, k_draw_suffix finishes the descents bucket by bucket on
-// XCD-affine blocks.  The arithmetic and comparisons are those of k_krp_draw,
-// so the results are identical.
-// ---------------------------------------------------------------------------
-template <int RMAX, int SG, int BS>
-__global__ void __launch_bounds__(BS) k_draw_prefix(DrawArgs a) {
-    using Cfg = DrawCfg<RMAX, SG>;
-    constexpr int EPL = Cfg::EPL, HPL = Cfg::HPL;
-    constexpr int GPW = 64 / SG;
-    __shared__ double lds_x[BS / SG][RMAX];
-    __shared__ uint16_t pair_tab[Cfg::TMAX];
-    fill_pairs<BS>(pair_tab, a.R);
-    const int lane = threadIdx.x & 63;
-    const int g = lane % SG;
-    const int wave = threadIdx.x / 64;
-    double* xs = lds_x[threadIdx.x / SG];
-    const int R = a.R;
-    const int T = (int)tri_size(R);
-    for (int b = g; b < RMAX; b += SG) xs[b] = 0.0;
-    wave_sync_lds();
-    const int mi = a.mi_begin;
-    const int k = a.order[mi];
-    const ModeDev& md = a.mode[k];
-    const uint64_t waves_total = (uint64_t)gridDim.x * (BS / 64);
-    const uint64_t n_items = (a.J + GPW - 1) / GPW;
-    for (uint64_t item = (uint64_t)blockIdx.x * (BS / 64) + wave; item < n_items; item += waves_total) {
-        const uint64_t i = item * GPW + lane / SG;
-        const bool active = i < a.J;
-        double h[HPL];
-#pragma unroll
-        for (int q = 0; q < HPL; q++) h[q] = 1.0;
-        if (mi > 0 && active) {
-#pragma unroll
-            for (int q = 0; q < HPL; q++)
-                if (g + SG * q < R) h[q] = a.h_state[i * R + g + SG * q];
-        }
-#pragma unroll
-        for (int q = 0; q < HPL; q++)
-            if (g + SG * q < R) xs[g + SG * q] = h[q];
-        wave_sync_lds();
-        double c64[EPL];
-        make_coefs<RMAX, SG>(xs, pair_tab, T, g, c64);
-        const double ue = active ? (a.draws ? a.draws[(uint64_t)k * a.J + i] : philox_uniform(a.seed, a.call, i, 2 * k))
-                                 : 0.5;
-        double low, high;
-        const uint64_t ce = descend<RMAX, SG, false>(md, a.esh, a.ts64, a.ts32, c64, md.etree, ue, g, low, high);
-        const uint64_t r = leaf_index(a.esh, ce);
-        wave_sync_lds();
-#pragma unroll
-        for (int q = 0; q < HPL; q++)
-            if (g + SG * q < R) {
-                const double x = h[q] * md.E[r * R + g + SG * q];
-                xs[g + SG * q] = x;
-                if (active) a.st_x[i * R + g + SG * q] = x;
-            }
-        wave_sync_lds();
-        make_coefs<RMAX, SG>(xs, pair_tab, T, g, c64);
-        const double ug = active ? (a.draws ? a.draws[(uint64_t)a.N * a.J + (uint64_t)k * a.J + i]
-                                            : philox_uniform(a.seed, a.call, i, 2 * k + 1))
-                                 : 0.5;
-        const double m = node_qform<double, EPL, SG>(md.tree64, c64, g, md.T);
-        uint64_t c = 0;
-        low = 0.0;
-        high = 1.0;
-        descend_steps<RMAX, SG, false>(md, md.sh, a.ts64, a.ts32, c64, md.tree64, ug, g, m, 0, a.split_level, false, c,
-                                       low, high);
-        if (active && g == 0) {
-            a.st_s[i * 4 + 0] = low;
-            a.st_s[i * 4 + 1] = high;
-            a.st_s[i * 4 + 2] = m;
-            a.st_s[i * 4 + 3] = (double)c;
-            a.bucket[i] = (uint32_t)(c - ((1ull << a.split_level) - 1)) % kBuckets;
-        }
-        wave_sync_lds();
-    }
-}
-
-// Stable partition of the samples by bucket (one block): list holds the
-// sample indices bucket by bucket, off[b] the start of bucket b.
-template <int BS>
-__global__ void __launch_bounds__(BS) k_bucket_partition(const uint32_t* __restrict__ bucket, uint64_t J,
-                                                         uint32_t* __restrict__ list, uint32_t* __restrict__ off) {
-    __shared__ uint32_t cnt[kBuckets][BS];
-    __shared__ uint32_t base[kBuckets + 1];
-    const uint32_t t = threadIdx.x;
-    const uint64_t chunk = (J + BS - 1) / BS;
-    const uint64_t s0 = min<uint64_t>(J, t * chunk), s1 = min<uint64_t>(J, s0 + chunk);
-    uint32_t c[kBuckets];
-#pragma unroll
-    for (uint32_t b = 0; b < kBuckets; b++) c[b] = 0;
-    for (uint64_t s = s0; s < s1; s++) c[bucket[s]]++;
-#pragma unroll
-    for (uint32_t b = 0; b < kBuckets; b++) cnt[b][t] = c[b];
-    __syncthreads();
-    if (t < kBuckets) {  // exclusive scan of bucket t over the threads
-        uint32_t run = 0;
-        for (uint32_t q = 0; q < BS; q++) {
-            const uint32_t v = cnt[t][q];
-            cnt[t][q] = run;
-            run += v;
-        }
-        base[t + 1] = run;  // size of bucket t
-    }
-    __syncthreads();
-    if (t == 0) {
-        uint32_t run = 0;
-        for (uint32_t b = 0; b < kBuckets; b++) {
-            const uint32_t n = base[b + 1];
-            base[b] = run;
-            run += n;
-            off[b] = base[b];
-        }
-        base[kBuckets] = run;
-        off[kBuckets] = run;
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t b = 0; b < kBuckets; b++) c[b] = base[b] + cnt[b][t];
-    for (uint64_t s = s0; s < s1; s++) list[c[bucket[s]]++] = (uint32_t)s;
-}
-
-template <int RMAX, int SG, int BS, bool USE32>
-__global__ void __launch_bounds__(BS) k_draw_suffix(DrawArgs a) {
-    using Cfg = DrawCfg<RMAX, SG>;
-    constexpr int EPL = Cfg::EPL, HPL = Cfg::HPL;
-    constexpr int GPW = 64 / SG;
-    __shared__ double lds_x[BS / SG][RMAX];
-    __shared__ double lds_q[BS / SG][RMAX];
-    __shared__ uint16_t pair_tab[Cfg::TMAX];
-    fill_pairs<BS>(pair_tab, a.R);
-    const int lane = threadIdx.x & 63;
-    const int g = lane % SG;
-    const int wave = threadIdx.x / 64;
-    double* xs = lds_x[threadIdx.x / SG];
-    double* qs = lds_q[threadIdx.x / SG];
-    const int R = a.R;
-    const int T = (int)tri_size(R);
-    for (int b = g; b < RMAX; b += SG) xs[b] = 0.0;
-    wave_sync_lds();
-    const int mi = a.mi_begin;
-    const int k = a.order[mi];
-    const ModeDev& md = a.mode[k];
-    const bool last = mi + 1 >= a.m;
-    const uint32_t bk = blockIdx.x % kBuckets;
-    const uint64_t nb = (gridDim.x + kBuckets - 1 - bk) / kBuckets;  // blocks serving bucket bk
-    const uint64_t sub = blockIdx.x / kBuckets;
-    const uint64_t b0 = a.boff[bk], n = a.boff[bk + 1] - b0;
-    const uint64_t waves_total = nb * (BS / 64);
-    const uint64_t n_items = (n + GPW - 1) / GPW;
-    for (uint64_t item = sub * (BS / 64) + wave; item < n_items; item += waves_total) {
-        const uint64_t t = item * GPW + lane / SG;
-        const bool active = t < n;
-        const uint64_t i = active ? a.blist[b0 + t] : 0;
-#pragma unroll
-        for (int q = 0; q < HPL; q++)
-            if (g + SG * q < R) xs[g + SG * q] = active ? a.st_x[i * R + g + SG * q] : 0.0;
-        wave_sync_lds();
-        double c64[EPL];
-        make_coefs<RMAX, SG>(xs, pair_tab, T, g, c64);
-        const double ug = active ? (a.draws ? a.draws[(uint64_t)a.N * a.J + (uint64_t)k * a.J + i]
-                                            : philox_uniform(a.seed, a.call, i, 2 * k + 1))
-                                 : 0.5;
-        double low = active ? a.st_s[i * 4 + 0] : 0.0;
-        double high = active ? a.st_s[i * 4 + 1] : 1.0;
-        const double m = active ? a.st_s[i * 4 + 2] : 1.0;
-        uint64_t c = active ? (uint64_t)a.st_s[i * 4 + 3] : ((1ull << a.split_level) - 1);
-        descend_steps<RMAX, SG, USE32>(md, md.sh, a.ts64, a.ts32, c64, md.tree64, ug, g, m, a.split_level,
-                                       (uint32_t)md.sh.lfill_level, true, c, low, high);
-        const uint64_t idx = leaf_index(md.sh, c);
-        uint32_t res = 0;
-        if (md.sh.F > 1) {
-            const double frac = (ug - low) / (high - low);
-            const uint64_t r0 = idx * md.sh.F;
-            const uint32_t rows = (uint32_t)min<uint64_t>(md.sh.F, md.sh.n - r0);
-            if constexpr (USE32)
-                res = leaf_scan<float, RMAX, SG>(md.U32, r0, rows, (uint32_t)md.sh.F, R, xs, qs, frac, g, lane);
-            else
-                res = leaf_scan<double, RMAX, SG>(md.U64, r0, rows, (uint32_t)md.sh.F, R, xs, qs, frac, g, lane);
-        }
-        const uint64_t srow = idx * md.sh.F + res;
-        double h[HPL];
-#pragma unroll
-        for (int q = 0; q < HPL; q++) {
-            h[q] = 1.0;
-            if (mi > 0 && active && g + SG * q < R) h[q] = a.h_state[i * R + g + SG * q];
-            if (g + SG * q < R) h[q] *= md.U64[srow * R + g + SG * q];
-        }
-        if (active && g == 0) a.samples[(uint64_t)k * a.J + i] = srow;
-        wave_sync_lds();
-        if (!last) {
-            if (active) {
-#pragma unroll
-                for (int q = 0; q < HPL; q++)
-                    if (g + SG * q < R) a.h_state[i * R + g + SG * q] = h[q];
-            }
-            continue;
-        }
-        // ---- weight: R / (J * h^T pinv h) (sampler.hpp:94-122) --------------
-#pragma unroll
-        for (int q = 0; q < HPL; q++)
-            if (g + SG * q < R) xs[g + SG * q] = h[q];
-        wave_sync_lds();
-        double part = 0.0;
-#pragma unroll
-        for (int q = 0; q < HPL; q++) {
-            const int ra = g + SG * q;
-            if (ra < R) {
-                double y = 0.0;
-                for (int b = 0; b < R; b++) y += a.pinv[ra * R + b] * xs[b];
-                part += h[q] * y;
-            }
-        }
-        const double lev = group_sum<SG>(part);
-        if (active) {
-            if (a.w_out && g == 0) a.w_out[i] = (double)R / (lev * (double)a.J);
-            if (a.h_out) {
-#pragma unroll
-                for (int q = 0; q < HPL; q++)
-                    if (g + SG * q < R) a.h_out[i * R + g + SG * q] = h[q];
-            }
-        }
-        wave_sync_lds();
     }
 }
 
