@@ -1078,10 +1078,13 @@ struct Als {
             lk->init(N, I, J, R, U, true, stream, kind == 2);
         } else {
             sampler = sampler_new_aliased(N, I, J, R, U, precision);
-            // after an update a long mode's factor is zero in all rows without a
-            // matched nonzero, and most samples descend to a few nodes that the
-            // caches hold anyway: ordering the samples only cost (5,700 against
-            // 5,609 us a sweep at 2^20 x 2^19 x 2^15, 2e7 nonzeros, R = 25)
+            // after an update a factor is zero in all rows without a matched
+            // nonzero and dominated by a few heavy ones: most samples descend to
+            // nodes that the caches hold anyway, and the others' paths follow
+            // their uniforms less.  Per sweep: ordered 5,700, in tiles 5,699,
+            // plain 5,540-5,609 us at 2^20 x 2^19 x 2^15, 2e7 nonzeros, R = 25;
+            // in tiles 6,417, plain 6,341 at 183 x 24 x 1140 x 1717.
+            sampler_set_option(sampler, "tile_descent", 0);
             sampler_set_option(sampler, "sample_order", 0);
         }
         samples = mem.alloc<uint64_t>(N * J);

@@ -19,6 +19,7 @@
 #include "ftl_common.hpp"
 #include "sampler_internal.hpp"
 #include "sampler_kernels.hpp"
+#include "tile_kernels.hpp"
 #include "tuning.hpp"
 
 namespace ftl {
@@ -437,6 +438,11 @@ struct Sampler {
     // option "sample_order": launches take the samples by increasing Gram
     // uniform (0 never, 1 always, 2 by order_pays)
     uint32_t sample_order = 2;
+    // option "tile_descent": eigen descents and upper Gram levels by the tile
+    // kernels (0 never, 1 always where they apply, 2 by tiles_pay)
+    uint32_t tile_descent = 2;
+    uint32_t* st_r = nullptr;
+    double* st_s = nullptr;
     uint16_t* order_bin = nullptr;
     uint32_t *order_count = nullptr, *order_perm = nullptr;
     double* h_state = nullptr;
@@ -754,6 +760,9 @@ struct Sampler {
         } else if (key == "sample_order") {
             FTL_REQUIRE(value >= 0 && value <= 2, "sample_order must be 0, 1 or 2");
             sample_order = (uint32_t)value;
+        } else if (key == "tile_descent") {
+            FTL_REQUIRE(value >= 0 && value <= 2, "tile_descent must be 0, 1 or 2");
+            tile_descent = (uint32_t)value;
         } else if (key == "xcd_buckets") {
             FTL_REQUIRE(value == 0 || value == 1, "xcd_buckets must be 0 or 1");
             sample_order = value ? 1 : 2;
@@ -833,6 +842,7 @@ struct Sampler {
         if (key == "block_threads") return block_threads;
         if (key == "overlap_compute_m") return overlap_cm && n_msets > 1;
         if (key == "sample_order") return sample_order;
+        if (key == "tile_descent") return tile_descent;
         if (key == "xcd_buckets") return sample_order == 1;
         if (key == "jacobi_threads") return jacobi_override ? jacobi_override : jacobi_threads_for(R);
         if (key == "fp32_levels") return fp32_levels;
@@ -964,9 +974,11 @@ struct Sampler {
         lam = msets[0].lam;
         h_state = dalloc<double>(J * R);
         if (J <= kOrderMaxJ) {
-            order_bin = dalloc<uint16_t>(N * J);
-            order_perm = dalloc<uint32_t>(N * J);
-            order_count = dalloc<uint32_t>(N * order_blocks(J) * kOrderBins);
+            order_bin = dalloc<uint16_t>(2 * N * J);
+            order_perm = dalloc<uint32_t>(2 * N * J);
+            order_count = dalloc<uint32_t>(2 * N * order_blocks(J) * kOrderBins);
+            st_r = dalloc<uint32_t>(J);
+            st_s = dalloc<double>(J * 4);
         }
         trees_dirty = true;
         if (sync_end) FTL_HIP_CHECK(hipStreamSynchronize(stream));
@@ -1004,7 +1016,9 @@ struct Sampler {
         total += up(R2 * 8) * 2 + up(N * R2 * 8) + up(((uint64_t)N * (2 * R - 1) * ts64 + pad) * 8) +
                  up((uint64_t)(N + 1) * 3 * (R + 1) * R * 8) + up((uint64_t)(N + 1) * R * 8);
         total += up(J * R * 8);
-        if (J <= kOrderMaxJ) total += up(N * J * 2) + up(N * J * 4) + up(N * order_blocks(J) * kOrderBins * 4);
+        if (J <= kOrderMaxJ)
+            total += up(2 * N * J * 2) + up(2 * N * J * 4) + up(2 * N * order_blocks(J) * kOrderBins * 4) + up(J * 4) +
+                     up(J * 4 * 8);
         return total;
     }
 
@@ -1065,23 +1079,23 @@ struct Sampler {
         if (evs) FTL_HIP_CHECK(hipEventRecord(evs[2], st));
     }
 
-    template <int RMAX, int SG, bool USE32>
+    template <int RMAX, int SG, bool USE32, bool RESUME>
     void launch_draw(const DrawArgs& a, hipStream_t st) {
         constexpr int BS = 256;
         const uint64_t per_block = BS / SG;
         uint64_t blocks = (J + per_block - 1) / per_block;
         if (grid_override) blocks = std::min<uint64_t>(blocks, grid_override);
         blocks = std::max<uint64_t>(1, std::min<uint64_t>(blocks, 1u << 20));
-        hipLaunchKernelGGL((k_krp_draw<RMAX, SG, BS, USE32>), dim3((unsigned)blocks), dim3(BS), 0, st, a);
+        hipLaunchKernelGGL((k_krp_draw<RMAX, SG, BS, USE32, RESUME>), dim3((unsigned)blocks), dim3(BS), 0, st, a);
         FTL_HIP_CHECK(hipGetLastError());
     }
 
-    template <int RMAX, int SG>
+    template <int RMAX, int SG, bool RESUME>
     void launch_draw_p(const DrawArgs& a, hipStream_t st) {
         if (precision == FTL_FP32)
-            launch_draw<RMAX, SG, true>(a, st);
+            launch_draw<RMAX, SG, true, RESUME>(a, st);
         else
-            launch_draw<RMAX, SG, false>(a, st);
+            launch_draw<RMAX, SG, false, RESUME>(a, st);
     }
 
     template <int RMAX, bool USE32>
@@ -1121,7 +1135,7 @@ struct Sampler {
 
     // One-sample-per-block kernel: a grid of as many blocks as are resident
     // at once, each looping over samples i = blockIdx.x + k * gridDim.x.
-    template <int RMAX, int BS, bool USE32>
+    template <int RMAX, int BS, bool USE32, bool RESUME>
     void launch_draw_block(const DrawArgs& a, hipStream_t st) {
         // blocks per CU and CU count, per instantiation (a function-local
         // static: initialised once, thread-safe; a throw leaves it unset)
@@ -1132,26 +1146,26 @@ struct Sampler {
             int dev = 0, cus = 0, nb = 0;
             FTL_HIP_CHECK(hipGetDevice(&dev));
             FTL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-            FTL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_krp_draw_block<RMAX, BS, USE32>, BS, 0));
+            FTL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_krp_draw_block<RMAX, BS, USE32, RESUME>, BS, 0));
             return Occ{std::max(1, nb), std::max(1, cus)};
         }();
         uint64_t blocks = std::min<uint64_t>(J, (uint64_t)occ.resident * (uint64_t)occ.cus);
         if (grid_override) blocks = std::min<uint64_t>(blocks, grid_override);
         blocks = std::max<uint64_t>(1, std::min<uint64_t>(blocks, 1u << 20));
-        hipLaunchKernelGGL((k_krp_draw_block<RMAX, BS, USE32>), dim3((unsigned)blocks), dim3(BS), 0, st, a);
+        hipLaunchKernelGGL((k_krp_draw_block<RMAX, BS, USE32, RESUME>), dim3((unsigned)blocks), dim3(BS), 0, st, a);
         FTL_HIP_CHECK(hipGetLastError());
     }
 
-    template <int RMAX, bool USE32>
+    template <int RMAX, bool USE32, bool RESUME>
     void launch_draw_block_bs(const DrawArgs& a, hipStream_t st) {
         const uint32_t bs = block_threads ? block_threads : 256u;
         if constexpr (RMAX == 64) {
-            if (bs == 128) launch_draw_block<64, 128, USE32>(a, st);
-            else launch_draw_block<64, 256, USE32>(a, st);
+            if (bs == 128) launch_draw_block<64, 128, USE32, RESUME>(a, st);
+            else launch_draw_block<64, 256, USE32, RESUME>(a, st);
         } else {
-            if (bs == 128) launch_draw_block<128, 128, USE32>(a, st);
-            else if (bs == 512) launch_draw_block<128, 512, USE32>(a, st);
-            else launch_draw_block<128, 256, USE32>(a, st);
+            if (bs == 128) launch_draw_block<128, 128, USE32, RESUME>(a, st);
+            else if (bs == 512) launch_draw_block<128, 512, USE32, RESUME>(a, st);
+            else launch_draw_block<128, 256, USE32, RESUME>(a, st);
         }
     }
 
@@ -1159,11 +1173,11 @@ struct Sampler {
         const uint32_t sg = sg_override;
         if ((draw_kernel == 2 && R > 32) || (draw_kernel == 0 && R > 64)) {
             if (R <= 64) {
-                if (precision == FTL_FP32) launch_draw_block_bs<64, true>(a, st);
-                else launch_draw_block_bs<64, false>(a, st);
+                if (precision == FTL_FP32) launch_draw_block_bs<64, true, false>(a, st);
+                else launch_draw_block_bs<64, false, false>(a, st);
             } else {
-                if (precision == FTL_FP32) launch_draw_block_bs<128, true>(a, st);
-                else launch_draw_block_bs<128, false>(a, st);
+                if (precision == FTL_FP32) launch_draw_block_bs<128, true, false>(a, st);
+                else launch_draw_block_bs<128, false, false>(a, st);
             }
             return;
         }
@@ -1180,7 +1194,59 @@ struct Sampler {
             }
             return;
         }
-        with_cfg([&](auto rmax, auto sgc) { launch_draw_p<decltype(rmax)::value, decltype(sgc)::value>(a, st); });
+        with_cfg([&](auto rmax, auto sgc) { launch_draw_p<decltype(rmax)::value, decltype(sgc)::value, false>(a, st); });
+    }
+
+    // When the modes of a call go through the tile kernels.  Draw kernels of a
+    // call against the group or block kernel in order: R = 128, I = 2^20, J =
+    // 50,000 FP32 7.7 / 13.8 ms; R = 65, I = 2^19 FP64 5.2 / 11.6 ms, J = 8192
+    // FP32 1.46 / 2.09 ms; R = 128, J = 8192 2.35 / 2.32 ms.  Up to R = 64 the
+    // group kernel reads a third as much per sample and a tile's chain of
+    // dependent matrix products is the longer one unless each SIMD has two
+    // tiles or more: J = 50,000, R = 33 1.56 / 2.23 ms, R = 64 2.11 / 2.47 ms, R
+    // = 32 (I = 2^22, two modes) 566 / 602 us, but J = 20,011, R = 64 1.14 / 1.09
+    // ms and J = 8192, R = 48 515 / 485 us.  R <= 16 leaves most of a 16 x 16
+    // block empty: 531 / 455 us.
+    bool tiles_pay() const { return R > 64 ? J >= 8192 : R > 16 && J >= 32768; }
+    bool tiled(const std::vector<int>& order) const {
+        if (!st_s || !mode_split || tile_descent == 0) return false;
+        for (int k : order)
+            if (modes[k].sh.node_count >= (1ull << 31)) return false;
+        return tile_descent == 1 || tiles_pay();
+    }
+
+    // One sampled mode: eigen rows, upper Gram levels, then the rest.
+    template <int NB>
+    void launch_tiles(DrawArgs a, hipStream_t st) {
+        const dim3 grid((unsigned)((J + 63) / 64));
+        const uint32_t* perm = order_perm + (uint64_t)a.mi_begin * J;
+        a.perm = perm + (uint64_t)a.m * J;
+        hipLaunchKernelGGL(k_tile_eigen<NB>, grid, dim3(256), 0, st, a);
+        FTL_HIP_CHECK(hipGetLastError());
+        a.perm = perm;
+        if (precision == FTL_FP32) hipLaunchKernelGGL((k_tile_gram<NB, true>), grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_tile_gram<NB, false>), grid, dim3(256), 0, st, a);
+        FTL_HIP_CHECK(hipGetLastError());
+    }
+
+    void dispatch_tiles(DrawArgs& a, hipStream_t st) {
+        switch ((R + 15) / 16) {
+            case 1: launch_tiles<1>(a, st); break;
+            case 2: launch_tiles<2>(a, st); break;
+            case 3: launch_tiles<3>(a, st); break;
+            case 4: launch_tiles<4>(a, st); break;
+            case 5: launch_tiles<5>(a, st); break;
+            case 6: launch_tiles<6>(a, st); break;
+            case 7: launch_tiles<7>(a, st); break;
+            default: launch_tiles<8>(a, st); break;
+        }
+        a.perm = order_perm + (uint64_t)a.mi_begin * J;
+        if (R > 64) {
+            if (precision == FTL_FP32) launch_draw_block_bs<128, true, true>(a, st);
+            else launch_draw_block_bs<128, false, true>(a, st);
+            return;
+        }
+        with_cfg([&](auto rmax, auto sgc) { launch_draw_p<decltype(rmax)::value, decltype(sgc)::value, true>(a, st); });
     }
 
     // When the order is made: nodes of 1.1 KB or more (R > 16), some tree of
@@ -1200,9 +1266,11 @@ struct Sampler {
     }
     bool ordered() const { return order_perm && (sample_order == 1 || (sample_order == 2 && order_pays())); }
 
-    // The order of every sampled mode's samples (k_order_*), queued on st.
-    void make_order(const std::vector<int>& order, const double* draws, hipStream_t st) {
+    // The orders of every sampled mode's samples (k_order_*) by their Gram
+    // uniforms and, with eigen, by their eigen uniforms, queued on st.
+    void make_order(const std::vector<int>& order, bool eigen, const double* draws, hipStream_t st) {
         OrderArgs o{};
+        o.m = (int)order.size();
         for (size_t t = 0; t < order.size(); t++) o.modes[t] = order[t];
         o.N = (int)N;
         o.J = J;
@@ -1213,7 +1281,7 @@ struct Sampler {
         o.bin = order_bin;
         o.count = order_count;
         o.perm = order_perm;
-        const dim3 grid((unsigned)order_blocks(J), (unsigned)order.size());
+        const dim3 grid((unsigned)order_blocks(J), (unsigned)order.size() * (eigen ? 2 : 1));
         hipLaunchKernelGGL(k_order_count, grid, dim3(256), 0, st, o);
         FTL_HIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(k_order_scatter, grid, dim3(256), 0, st, o);
@@ -1251,6 +1319,8 @@ struct Sampler {
         a.pinv = ms.pinv;
         a.leaf32 = (int)leaf32;
         a.draws = draws;
+        a.st_r = st_r;
+        a.st_s = st_s;
         a.seed = seed;
         a.call = call;
         a.samples = samples;
@@ -1278,7 +1348,8 @@ struct Sampler {
         if (timing)
             for (auto& e : evs) e = take_event();
         const bool overlap = overlap_cm && n_msets > 1;
-        const bool by_order = ordered();
+        const bool tiles = tiled(order);
+        const bool by_order = tiles || ordered();
         const MSet& ms = msets[overlap ? (mset_next++ & 1) : 0];
         if (overlap) {
             if (trees_dirty) {
@@ -1289,10 +1360,10 @@ struct Sampler {
             FTL_HIP_CHECK(hipStreamWaitEvent(cm_stream, ms.draw_done, 0));
             compute_m(j, cm_stream, ms, timing ? evs.data() : nullptr);
             FTL_HIP_CHECK(hipEventRecord(ms.cm_done, cm_stream));
-            if (by_order) make_order(order, draws, st);
+            if (by_order) make_order(order, tiles, draws, st);
             FTL_HIP_CHECK(hipStreamWaitEvent(st, ms.cm_done, 0));
         } else {
-            if (by_order) make_order(order, draws, st);
+            if (by_order) make_order(order, tiles, draws, st);
             compute_m(j, st, ms, timing ? evs.data() : nullptr);
         }
         if (timing) FTL_HIP_CHECK(hipEventRecord(evs[3], st));
@@ -1302,6 +1373,10 @@ struct Sampler {
             for (int mi = 0; mi < a.m; mi++) {
                 a.mi_begin = mi;
                 a.mi_end = mi + 1;
+                if (tiles) {
+                    dispatch_tiles(a, st);
+                    continue;
+                }
                 a.perm = by_order ? order_perm + (uint64_t)mi * J : nullptr;
                 dispatch_draw(a, st);
             }

@@ -837,6 +837,10 @@ struct DrawArgs {
     // the order in which the launch goes through the samples (J indices, by
     // k_order_*), or null for 0..J-1
     const uint32_t* perm;
+    // a mode's launches in tiles (tile_kernels.hpp): eigen row of each sample,
+    // and {low, high, m, level << 32 | node} where its Gram descent goes on
+    uint32_t* st_r;
+    double* st_s;      // J x 4
 };
 
 // ---------------------------------------------------------------------------
@@ -853,7 +857,7 @@ struct DrawArgs {
 // sum the table up to their own entries (device-scope atomics on one table
 // took 34 us for three modes of 50,000 samples, most of it their round trips).
 // ---------------------------------------------------------------------------
-constexpr uint32_t kOrderBins = 2048;
+constexpr uint32_t kOrderBins = 4096;
 constexpr uint32_t kOrderMaxBlocks = 256;
 constexpr uint32_t kXcds = 8;
 
@@ -864,15 +868,18 @@ __host__ __device__ inline uint32_t order_share(uint64_t J) {
 }
 
 struct OrderArgs {
-    int modes[kMaxModes];  // sampled modes; blockIdx.y is the position
+    // one order per row (blockIdx.y): of the Gram uniforms of the m sampled
+    // modes, then, when gridDim.y = 2 m, of their eigen uniforms
+    int modes[kMaxModes];
+    int m;
     int N;
     uint64_t J;
     uint32_t share;        // order_share(J); gridDim.x = ceil(J / share)
     const double* draws;   // 2*N*J or null (Philox)
     uint64_t seed, call;
-    uint16_t* bin;         // m x J
-    uint32_t* count;       // m x gridDim.x x kOrderBins
-    uint32_t* perm;        // m x J
+    uint16_t* bin;         // rows x J
+    uint32_t* count;       // rows x gridDim.x x kOrderBins
+    uint32_t* perm;        // rows x J
 };
 
 __global__ void __launch_bounds__(256) k_order_count(OrderArgs a) {
@@ -880,12 +887,13 @@ __global__ void __launch_bounds__(256) k_order_count(OrderArgs a) {
     for (uint32_t b = threadIdx.x; b < kOrderBins; b += 256) cnt[b] = 0;
     __syncthreads();
     const uint32_t t = blockIdx.y;
-    const int k = a.modes[t];
+    const int gram = (int)t < a.m ? 1 : 0;
+    const int k = a.modes[gram ? t : t - a.m];
     const uint64_t i0 = (uint64_t)blockIdx.x * a.share, i1 = min(i0 + a.share, a.J);
-    const double* u_given = a.draws ? a.draws + ((uint64_t)a.N + k) * a.J : nullptr;
+    const double* u_given = a.draws ? a.draws + ((uint64_t)(gram ? a.N : 0) + k) * a.J : nullptr;
 #pragma unroll 8
     for (uint64_t i = i0 + threadIdx.x; i < i1; i += 256) {
-        const double u = u_given ? u_given[i] : philox_uniform(a.seed, a.call, i, 2 * k + 1);
+        const double u = u_given ? u_given[i] : philox_uniform(a.seed, a.call, i, 2 * k + gram);
         const uint32_t b = u >= 1.0 ? kOrderBins - 1 : u > 0.0 ? (uint32_t)(u * kOrderBins) : 0u;
         a.bin[t * a.J + i] = (uint16_t)b;
         atomicAdd(cnt + b, 1u);
@@ -908,14 +916,16 @@ __global__ void __launch_bounds__(256) k_order_scatter(OrderArgs a) {
     const uint32_t* src = a.count + (uint64_t)t * gridDim.x * kOrderBins + threadIdx.x * PT;
 #pragma unroll 4
     for (uint32_t b = 0; b < gridDim.x; b++) {
-        const uint4 c0 = *reinterpret_cast<const uint4*>(src + b * kOrderBins);
-        const uint4 c1 = *reinterpret_cast<const uint4*>(src + b * kOrderBins + 4);
-        const uint32_t c[PT] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
         const uint32_t own = b < blockIdx.x ? ~0u : 0u;
 #pragma unroll
-        for (int q = 0; q < PT; q++) {
-            all[q] += c[q];
-            before[q] += c[q] & own;
+        for (int q = 0; q < PT; q += 4) {
+            const uint4 c = *reinterpret_cast<const uint4*>(src + b * kOrderBins + q);
+            const uint32_t v[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                all[q + e] += v[e];
+                before[q + e] += v[e] & own;
+            }
         }
     }
     uint32_t run = 0;
@@ -1092,18 +1102,16 @@ __device__ inline uint64_t descend(const ModeDev& md, const Shape& sh, uint32_t 
     return c;
 }
 
-// Descent steps d_begin .. d_end-1 (and the guarded tail level when tail)
-// from the state (c, low, high) with root mass m: the loop of descend, split
-// so that a descent can stop after the top levels and resume elsewhere.
+// The rest of a descent that stands at node c of level d0 (d0 <= lfill_level).
 template <int RMAX, int SG, bool USE32>
-__device__ inline void descend_steps(const ModeDev& md, const Shape& sh, uint32_t ts64, uint32_t ts32,
-                                     const double (&c64)[DrawCfg<RMAX, SG>::EPL], const double* tree64, double u,
-                                     int g, double m, uint32_t d_begin, uint32_t d_end, bool tail, uint64_t& c,
-                                     double& low, double& high) {
+__device__ inline void descend_from(const ModeDev& md, const Shape& sh, uint32_t ts64, uint32_t ts32,
+                                    const double (&c64)[DrawCfg<RMAX, SG>::EPL], double u, int g, double m,
+                                    uint32_t d0, uint64_t& c, double& low, double& high) {
     constexpr int EPL = DrawCfg<RMAX, SG>::EPL;
-    for (uint32_t d = d_begin; d < d_end; d++) {
+    for (uint32_t d = d0; d <= sh.lfill_level; d++) {
         const uint64_t child = 2 * c + 1;
-        const double mL = child_qform<EPL, SG, USE32>(md, tree64, child, d + 1, ts64, ts32, c64, g);
+        if (child >= sh.node_count) break;  // a leaf on the lfill level
+        const double mL = child_qform<EPL, SG, USE32>(md, md.tree64, child, d + 1, ts64, ts32, c64, g);
         const double cutoff = low + mL / m;
         if (u <= cutoff) {
             c = child;
@@ -1111,22 +1119,6 @@ __device__ inline void descend_steps(const ModeDev& md, const Shape& sh, uint32_
         } else {
             c = child + 1;
             low = cutoff;
-        }
-    }
-    if (tail && sh.node_count > sh.nodes_before_lfill) {
-        const bool leaf = 2 * c + 1 >= sh.node_count;
-        if (!leaf) {
-            const uint64_t child = 2 * c + 1;
-            const double mL =
-                child_qform<EPL, SG, USE32>(md, tree64, child, (uint32_t)sh.lfill_level + 1, ts64, ts32, c64, g);
-            const double cutoff = low + mL / m;
-            if (u <= cutoff) {
-                c = child;
-                high = cutoff;
-            } else {
-                c = child + 1;
-                low = cutoff;
-            }
         }
     }
 }
@@ -1234,7 +1226,8 @@ __device__ inline uint32_t leaf_scan(const TU* __restrict__ U, uint64_t r0, uint
 // in [a.mi_begin, a.mi_end), then the weight when the launch ends the draw).
 // xs / qs: the group's x and leaf-scan buffers in LDS; pair_tab: the packed
 // (row, column) table of a.R.
-template <int RMAX, int SG, bool USE32>
+// RESUME: the eigen row and the upper Gram levels come from the tile kernels.
+template <int RMAX, int SG, bool USE32, bool RESUME>
 __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, double* xs, double* qs,
                                               const uint16_t* pair_tab, int lane, int g) {
     using Cfg = DrawCfg<RMAX, SG>;
@@ -1258,19 +1251,24 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
     for (int mi = a.mi_begin; mi < a.mi_end; mi++) {
         const int k = a.order[mi];
         const ModeDev& md = a.mode[k];
+        double c64[EPL];
+        double low, high;
+        uint64_t r;
+        if constexpr (RESUME) {
+            r = active ? a.st_r[i] : 0;
+        } else {
         // ---- eigen stage: x = h -----------------------------------------
 #pragma unroll
         for (int q = 0; q < HPL; q++)
             if (g + SG * q < R) xs[g + SG * q] = h[q];
         wave_sync_lds();
-        double c64[EPL];
         make_coefs<RMAX, SG>(xs, pair_tab, T, g, c64);
         double ue = active ? (a.draws ? a.draws[(uint64_t)k * a.J + i] : philox_uniform(a.seed, a.call, i, 2 * k))
                            : 0.5;
-        double low, high;
         const uint64_t ce = descend<RMAX, SG, false>(md, a.esh, a.ts64, a.ts32, c64, md.etree, ue, g, low, high);
-        const uint64_t r = leaf_index(a.esh, ce);
+        r = leaf_index(a.esh, ce);
         wave_sync_lds();
+        }
         // scaled_h = h (.) E_k[r]
 #pragma unroll
         for (int q = 0; q < HPL; q++)
@@ -1281,8 +1279,21 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
         const double ug = active ? (a.draws ? a.draws[(uint64_t)a.N * a.J + (uint64_t)k * a.J + i]
                                             : philox_uniform(a.seed, a.call, i, 2 * k + 1))
                                  : 0.5;
-        const uint64_t c = descend<RMAX, SG, fp32>(md, md.sh, a.ts64, a.ts32, c64, md.tree64, ug, g, low, high);
-        const uint64_t idx = leaf_index(md.sh, c);
+        uint64_t c;
+        if constexpr (RESUME) {
+            const double* st = a.st_s + i * 4;
+            const uint64_t at = active ? (uint64_t)__double_as_longlong(st[3]) : 0;
+            low = active ? st[0] : 0.0;
+            high = active ? st[1] : 1.0;
+            c = at & 0xffffffffu;
+            descend_from<RMAX, SG, fp32>(md, md.sh, a.ts64, a.ts32, c64, ug, g, active ? st[2] : 1.0,
+                                         active ? (uint32_t)(at >> 32) : (uint32_t)md.sh.lfill_level + 1, c, low,
+                                         high);
+        } else {
+            c = descend<RMAX, SG, fp32>(md, md.sh, a.ts64, a.ts32, c64, md.tree64, ug, g, low, high);
+        }
+        // an inactive group scans the first leaf and writes nothing
+        const uint64_t idx = active || !RESUME ? leaf_index(md.sh, c) : 0;
         uint32_t res = 0;
         if (md.sh.F > 1) {
             const double frac = (ug - low) / (high - low);
@@ -1335,7 +1346,7 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
     wave_sync_lds();
 }
 
-template <int RMAX, int SG, int BS, bool USE32>
+template <int RMAX, int SG, int BS, bool USE32, bool RESUME>
 __global__ void __launch_bounds__(BS) k_krp_draw(DrawArgs a) {
     using Cfg = DrawCfg<RMAX, SG>;
     constexpr int GPW = 64 / SG;  // groups per wave
@@ -1357,7 +1368,7 @@ __global__ void __launch_bounds__(BS) k_krp_draw(DrawArgs a) {
     const uint64_t wave_id = (uint64_t)block * (BS / 64) + wave;
     const uint64_t n_items = (a.J + GPW - 1) / GPW;
     for (uint64_t item = wave_id; item < n_items; item += waves_total)
-        krp_draw_item<RMAX, SG, USE32>(a, item, xs, qs, pair_tab, lane, g);
+        krp_draw_item<RMAX, SG, USE32, RESUME>(a, item, xs, qs, pair_tab, lane, g);
 }
 
 // Packed draw of several requests (the same R and precision) in one launch:
@@ -1394,7 +1405,7 @@ __global__ void __launch_bounds__(BS) k_krp_draw_packed(const DrawArgs* __restri
             else hi = mid;
         }
         const uint32_t r = (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
-        krp_draw_item<RMAX, SG, USE32>(reqs[r], item - item_off[r], xs, qs, pair_tab, lane, g);
+        krp_draw_item<RMAX, SG, USE32, false>(reqs[r], item - item_off[r], xs, qs, pair_tab, lane, g);
     }
 }
 
@@ -1617,17 +1628,13 @@ __device__ inline double child_qform_block(const ModeDev& md, const double* tree
 }
 
 // The inverse-CDF descent of descend (partition_tree.hpp:251-332) with
-// block-wide node masses.
+// block-wide node masses, from node c of level d0 on; m: the root mass.
 template <int EPL, int BS, bool USE32>
-__device__ inline uint64_t descend_block(const ModeDev& md, const Shape& sh, uint32_t ts64, uint32_t ts32,
-                                         const double (&c64)[EPL], const double* tree64, double u, double* red,
-                                         int& par, double& low, double& high) {
-    const double m = node_qform_block<double, EPL, BS>(tree64, c64, red, par, md.T);
-    uint64_t c = 0;
-    low = 0.0;
-    high = 1.0;
+__device__ inline void descend_block(const ModeDev& md, const Shape& sh, uint32_t ts64, uint32_t ts32,
+                                     const double (&c64)[EPL], const double* tree64, double u, double* red, int& par,
+                                     double m, uint32_t d0, uint64_t& c, double& low, double& high) {
     const uint32_t levels = sh.lfill_level + ((sh.node_count > sh.nodes_before_lfill) ? 1u : 0u);
-    for (uint32_t d = 0; d < levels; d++) {
+    for (uint32_t d = d0; d < levels; d++) {
         // the guarded tail level (partition_tree.hpp:304-332): a leaf on the
         // lfill level stops the descent
         if (d == sh.lfill_level && 2 * c + 1 >= sh.node_count) break;
@@ -1642,7 +1649,6 @@ __device__ inline uint64_t descend_block(const ModeDev& md, const Shape& sh, uin
             low = cutoff;
         }
     }
-    return c;
 }
 
 // Leaf scan of one sample with the whole block (partition_tree.hpp:336-391):
@@ -1732,7 +1738,7 @@ __device__ inline uint32_t leaf_scan_block(const TU* __restrict__ U, uint64_t r0
     return res;
 }
 
-template <int RMAX, int BS, bool USE32>
+template <int RMAX, int BS, bool USE32, bool RESUME>
 __global__ void __launch_bounds__(BS) k_krp_draw_block(DrawArgs a) {
     static_assert(BS >= RMAX && BS % 64 == 0, "one h entry per thread");
     using Cfg = DrawCfg<RMAX, BS>;
@@ -1767,16 +1773,23 @@ __global__ void __launch_bounds__(BS) k_krp_draw_block(DrawArgs a) {
         for (int mi = a.mi_begin; mi < a.mi_end; mi++) {
             const int k = a.order[mi];
             const ModeDev& md = a.mode[k];
-            // ---- eigen stage: x = h -----------------------------------------
-            if (tid < R) xs[tid] = h;
-            __syncthreads();
             double c64[EPL];
-            make_coefs<RMAX, BS>(xs, pair_tab, T, tid, c64);
-            const double ue = a.draws ? a.draws[(uint64_t)k * a.J + i] : philox_uniform(a.seed, a.call, i, 2 * k);
-            double low, high;
-            const uint64_t ce = descend_block<EPL, BS, false>(md, a.esh, a.ts64, a.ts32, c64, md.etree, ue, red, par,
-                                                              low, high);
-            const uint64_t r = leaf_index(a.esh, ce);
+            double low = 0.0, high = 1.0;
+            uint64_t c = 0;
+            uint64_t r;
+            if constexpr (RESUME) {
+                r = a.st_r[i];
+            } else {
+                // ---- eigen stage: x = h -------------------------------------
+                if (tid < R) xs[tid] = h;
+                __syncthreads();
+                make_coefs<RMAX, BS>(xs, pair_tab, T, tid, c64);
+                const double ue = a.draws ? a.draws[(uint64_t)k * a.J + i] : philox_uniform(a.seed, a.call, i, 2 * k);
+                const double me = node_qform_block<double, EPL, BS>(md.etree, c64, red, par, md.T);
+                descend_block<EPL, BS, false>(md, a.esh, a.ts64, a.ts32, c64, md.etree, ue, red, par, me, 0, c, low,
+                                              high);
+                r = leaf_index(a.esh, c);
+            }
             // every thread has passed the descent's barriers after its
             // make_coefs reads of xs
             if (tid < R) xs[tid] = h * md.E[r * R + tid];
@@ -1785,8 +1798,23 @@ __global__ void __launch_bounds__(BS) k_krp_draw_block(DrawArgs a) {
             make_coefs<RMAX, BS>(xs, pair_tab, T, tid, c64);
             const double ug = a.draws ? a.draws[(uint64_t)a.N * a.J + (uint64_t)k * a.J + i]
                                       : philox_uniform(a.seed, a.call, i, 2 * k + 1);
-            const uint64_t c = descend_block<EPL, BS, USE32>(md, md.sh, a.ts64, a.ts32, c64, md.tree64, ug, red, par,
-                                                             low, high);
+            double m;
+            uint32_t d0 = 0;
+            if constexpr (RESUME) {
+                const double* st = a.st_s + i * 4;
+                const uint64_t at = (uint64_t)__double_as_longlong(st[3]);
+                low = st[0];
+                high = st[1];
+                m = st[2];
+                c = at & 0xffffffffu;
+                d0 = (uint32_t)(at >> 32);
+            } else {
+                m = node_qform_block<double, EPL, BS>(md.tree64, c64, red, par, md.T);
+                c = 0;
+                low = 0.0;
+                high = 1.0;
+            }
+            descend_block<EPL, BS, USE32>(md, md.sh, a.ts64, a.ts32, c64, md.tree64, ug, red, par, m, d0, c, low, high);
             const uint64_t idx = leaf_index(md.sh, c);
             uint32_t res = 0;
             if (md.sh.F > 1) {
