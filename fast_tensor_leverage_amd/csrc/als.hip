@@ -759,7 +759,7 @@ struct LKSampler {
         const uint32_t T = r * (r + 1) / 2;
         hipLaunchKernelGGL(k_partials_to8, dim3((8 * T + 255) / 256), dim3(256), 0, stream, gparts, nb, T, gred);
         FTL_LAUNCH_CHECK();
-        const uint64_t jac = 3 * (R + 1) * R <= (uint64_t)kJacobiLdsDoubles ? 3 * (R + 1) * R : (R + 1) * R;
+        const uint64_t jac = jacobi_lds_doubles(R);
         hipLaunchKernelGGL(k_pinv_partials<1024>, dim3(1), dim3(1024), jac * sizeof(double), stream, gred, 8u,
                            counters, r, pinv, work, lam);
         FTL_LAUNCH_CHECK();
@@ -1182,7 +1182,7 @@ struct Als {
                            J, (uint32_t)R, h, w, hs, hdd);
         FTL_LAUNCH_CHECK();
         gram_partials(hs, mt.counters + kCntUnique, 0, gpart, kGramBlocks);
-        const uint64_t jac = 3 * (R + 1) * R <= (uint64_t)kJacobiLdsDoubles ? 3 * (R + 1) * R : (R + 1) * R;
+        const uint64_t jac = jacobi_lds_doubles(R);
         if (jacobi_threads_for(R) == 256)
             hipLaunchKernelGGL(k_pinv_partials<256>, dim3(1), dim3(256), jac * sizeof(double), st, gpart,
                                kGramBlocks, mt.counters, (uint32_t)R, pinv, work, lam);
@@ -1287,7 +1287,7 @@ struct Als {
         hipLaunchKernelGGL(k_gram_hadamard, dim3(grid_for(T, 256)), dim3(256), 0, st, gram_red, N, (uint32_t)T, j,
                            gram_had);
         FTL_LAUNCH_CHECK();
-        const uint64_t jac = 3 * (R + 1) * R <= (uint64_t)kJacobiLdsDoubles ? 3 * (R + 1) * R : (R + 1) * R;
+        const uint64_t jac = jacobi_lds_doubles(R);
         if (jacobi_threads_for(R) == 256)
             hipLaunchKernelGGL(k_pinv_partials<256>, dim3(1), dim3(256), jac * sizeof(double), st, gram_had, 1u,
                                full_rank, (uint32_t)R, pinv, work, lam);

@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(BS) k_gram_partial(const double* __restrict__ 
 // v >= R - target and lambda_v > 1e-11 with target = min(J', R), then
 // pinv = M' M'^T with M'[:, v] = V[:, v] / sqrt(lambda_v) (common.h:228-323).
 // One block; pinv written full symmetric (R x R).
-// pinv of a symmetric R x R matrix A (LDS, leading dimension R + 1) as its
+// pinv of a symmetric R x R matrix A (LDS, leading dimension jacobi_ld(R)) as its
 // inverse by Cholesky, when that equals the eigendecomposition-based pinv
 // with the 1e-11 cut at full target rank (compute_pinv_square,
 // common.h:228-269): lambda_min(A) >= 1 / ||A^-1||_F > 2e-11 certifies that
@@ -312,10 +312,10 @@ __device__ bool pinv_cholesky(const double* A, double* C, double* Li, int R, dou
 #pragma clang fp contract(off)
     __shared__ double red[BS];
     __shared__ int fail;
-    const int tid = threadIdx.x, LD = R + 1;
+    const int tid = threadIdx.x, LD = R + 1, LDA = jacobi_ld(R);
     for (int e = tid; e < R * R; e += BS) {
         const int i = e / R, j = e - i * R;
-        C[i * LD + j] = A[i * LD + j];
+        C[i * LD + j] = A[i * LDA + j];
     }
     if (tid == 0) fail = 0;
     __syncthreads();
@@ -354,7 +354,7 @@ __device__ bool pinv_cholesky(const double* A, double* C, double* Li, int R, dou
         for (int m = m0; m < R; m++) s = s + Li[m * R + a] * Li[m * R + b];
         pinv[e] = s;
         f_inv = f_inv + s * s;
-        const double x = A[a * LD + b];
+        const double x = A[a * LDA + b];
         f_a = f_a + x * x;
         if (!(s == s) || s - s != 0.0) fail = 1;  // NaN or infinity
     }
@@ -388,8 +388,10 @@ __global__ void __launch_bounds__(BS) k_pinv_partials(const double* __restrict__
     __shared__ JacobiShared js;
     __shared__ double lam[128], diag_tmp[128];
     const int tid = threadIdx.x;
-    const int Ri = (int)R, LD = Ri + 1, T = Ri * (Ri + 1) / 2;
+    const int Ri = (int)R, LD = jacobi_ld(Ri), T = Ri * (Ri + 1) / 2;
     JacobiStore st = jacobi_store(smem, work, Ri);
+    if (jacobi_n2(Ri) > Ri && Ri <= kJacobiSmallR)
+        for (int e = tid; e <= Ri; e += BS) st.A[e * LD + Ri] = st.A[Ri * LD + e] = 0.0;
     for (int e = tid; e < T; e += BS) {
         // packed index e -> (a, b), a <= b
         int a = 0, base = 0;
@@ -416,10 +418,10 @@ __global__ void __launch_bounds__(BS) k_pinv_partials(const double* __restrict__
     const uint32_t Jp = counters[kCntUnique];
     const int target = (int)min<uint32_t>(Jp, R);
     // full target rank and a well-conditioned Gram: pinv = G^-1 by Cholesky
-    if (target == Ri && Ri <= kCholMaxR && 3 * LD * Ri <= kJacobiLdsDoubles &&
+    if (target == Ri && Ri <= kCholMaxR && Ri <= kJacobiSmallR &&
         pinv_cholesky<BS>(st.A, st.V, st.vecs, Ri, pinv))
         return;
-    jacobi_block<BS>(st.A, st.V, Ri, lam, st.vecs, js, diag_tmp);
+    jacobi_block<BS>(st, Ri, lam, js, diag_tmp);
     // M' in place of the eigenvectors
     for (int w = tid; w < Ri * Ri; w += BS) {
         const int u = w / Ri, v = w - u * Ri;

@@ -387,7 +387,9 @@ struct Sampler {
     // next computeM into the set after the draw that read it, and trees_ev
     // every computeM after the tree builds queued before it.
     struct MSet {
-        double *pinv = nullptr, *W = nullptr, *E = nullptr, *etree = nullptr, *work = nullptr, *lam = nullptr;
+        double *pinv = nullptr, *W = nullptr, *E = nullptr, *etree = nullptr, *lam = nullptr;
+        double* log = nullptr;
+        int* rank = nullptr;
         hipEvent_t cm_done = nullptr, draw_done = nullptr;
     };
     MSet msets[2];
@@ -416,7 +418,7 @@ struct Sampler {
     // option "overlap_compute_m" (only with a stream of the sampler's own)
     uint32_t overlap_cm = 1;
     // set 0 (compute_m_host and the single-set samplers read these)
-    double *pinv = nullptr, *W = nullptr, *E = nullptr, *etree = nullptr, *work = nullptr, *lam = nullptr;
+    double *pinv = nullptr, *W = nullptr, *E = nullptr, *etree = nullptr, *lam = nullptr;
     uint32_t etree_nodes = 0;
     // staging for the host-pointer API
     uint64_t* samples_dev = nullptr;
@@ -907,16 +909,20 @@ struct Sampler {
                                 (const void*)k_subtree_pairs<3>,     (const void*)k_subtree_pairs<4>};
             for (const void* f : sb)
                 FTL_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSubtreeLds));
-            // computeM blocks hold A ((R+1) R doubles) in LDS, plus V and the
-            // eigenvectors when R <= 64: at most 132 KB of dynamic LDS
+            // computeM blocks hold A twice and V in LDS (R < kJacobiSplitR), or
+            // A, twice up to R = 96 (149 KB)
             const void* cm[] = {(const void*)k_gram_pinv<256>, (const void*)k_eigen_modes<256>,
                                 (const void*)k_gram_pinv<512>, (const void*)k_eigen_modes<512>,
                                 (const void*)k_gram_pinv<1024>, (const void*)k_eigen_modes<1024>,
                                 (const void*)k_gram_pinv_batched<256>, (const void*)k_eigen_modes_batched<256>,
                                 (const void*)k_gram_pinv_batched<512>, (const void*)k_eigen_modes_batched<512>,
-                                (const void*)k_gram_pinv_batched<1024>, (const void*)k_eigen_modes_batched<1024>};
+                                (const void*)k_gram_pinv_batched<1024>, (const void*)k_eigen_modes_batched<1024>,
+                                (const void*)k_cm_solve<256, true>, (const void*)k_cm_solve<512, true>,
+                                (const void*)k_cm_solve<1024, true>, (const void*)k_cm_solve<256, false>,
+                                (const void*)k_cm_solve<512, false>, (const void*)k_cm_solve<1024, false>,
+                                (const void*)k_cm_etree};
             for (const void* f : cm)
-                FTL_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 129 * 128 * 8));
+                FTL_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 97 * 96 * 2 * 8));
         });
         // Tail pad of every tree: the draw kernels read 2 SG ceil(Tmax/(2 SG))
         // entries from a node start (SG up to 512 lanes per sample), Tmax
@@ -954,7 +960,10 @@ struct Sampler {
             ms.W = dalloc<double>(R2);
             ms.E = dalloc<double>(N * R2);
             ms.etree = dalloc<double>((uint64_t)N * etree_nodes * ts64 + pad);
-            ms.work = dalloc<double>((uint64_t)(N + 1) * 3 * (R + 1) * R);
+            if (R >= (uint64_t)kJacobiSplitR) {
+                ms.log = dalloc<double>((N + 1) * jacobi_log_doubles(R));
+                ms.rank = dalloc<int>((N + 1) * (R + 1));
+            }
             ms.lam = dalloc<double>((uint64_t)(N + 1) * R);
             FTL_HIP_CHECK(hipMemsetAsync(ms.E, 0, N * R2 * sizeof(double), stream));
             FTL_HIP_CHECK(
@@ -970,7 +979,6 @@ struct Sampler {
         W = msets[0].W;
         E = msets[0].E;
         etree = msets[0].etree;
-        work = msets[0].work;
         lam = msets[0].lam;
         h_state = dalloc<double>(J * R);
         if (J <= kOrderMaxJ) {
@@ -1014,7 +1022,9 @@ struct Sampler {
         }
         const uint64_t R2 = R * R;
         total += up(R2 * 8) * 2 + up(N * R2 * 8) + up(((uint64_t)N * (2 * R - 1) * ts64 + pad) * 8) +
-                 up((uint64_t)(N + 1) * 3 * (R + 1) * R * 8) + up((uint64_t)(N + 1) * R * 8);
+                 up((uint64_t)(N + 1) * R * 8);
+        if (R >= (uint64_t)kJacobiSplitR)
+            total += up((N + 1) * jacobi_log_doubles(R) * 8) + up((N + 1) * (R + 1) * sizeof(int));
         total += up(J * R * 8);
         if (J <= kOrderMaxJ)
             total += up(2 * N * J * 2) + up(2 * N * J * 4) + up(2 * N * order_blocks(J) * kOrderBins * 4) + up(J * 4) +
@@ -1049,7 +1059,8 @@ struct Sampler {
         a.W = ms.W;
         a.E = ms.E;
         a.etree = ms.etree;
-        a.work = ms.work;
+        a.log = reinterpret_cast<double2*>(ms.log);
+        a.rank = ms.rank;
         a.lam_out = ms.lam;
         a.ts64 = ts64;
         a.etree_nodes = etree_nodes;
@@ -1060,21 +1071,65 @@ struct Sampler {
         std::vector<int> order = sampled_modes(j);
         FTL_REQUIRE(!order.empty(), "no mode left to sample (N == 1 and j == 0)");
         ComputeMArgs a = computeM_args(order, ms);
-        const uint64_t jac = 3 * (R + 1) * R <= (uint64_t)kJacobiLdsDoubles ? 3 * (R + 1) * R : (R + 1) * R;
-        const size_t lds = jac * sizeof(double);
-        const uint32_t bs = jacobi_override ? jacobi_override : jacobi_threads_for(R);
-        if (bs == 256) launch_cm<256>(a, lds, st, evs);
-        else if (bs == 512) launch_cm<512>(a, lds, st, evs);
-        else launch_cm<1024>(a, lds, st, evs);
+        const uint32_t bs = jacobi_threads();
+        if (R >= (uint64_t)kJacobiSplitR) {
+            ComputeMSel sel{};
+            sel.one = a;
+            launch_cm_split(sel, 1, (uint32_t)a.m, st, evs);
+        } else if (bs == 256) {
+            launch_cm<256>(a, st, evs);
+        } else if (bs == 512) {
+            launch_cm<512>(a, st, evs);
+        } else {
+            launch_cm<1024>(a, st, evs);
+        }
     }
 
+    uint32_t jacobi_threads() const { return jacobi_override ? jacobi_override : jacobi_threads_for(R); }
+
     template <int BS>
-    void launch_cm(const ComputeMArgs& a, size_t lds, hipStream_t st, hipEvent_t* evs) {
+    void launch_cm(const ComputeMArgs& a, hipStream_t st, hipEvent_t* evs) {
+        const size_t lds = jacobi_lds_doubles(R) * sizeof(double);
         if (evs) FTL_HIP_CHECK(hipEventRecord(evs[0], st));
         hipLaunchKernelGGL(k_gram_pinv<BS>, dim3(1), dim3(BS), lds, st, a);
         FTL_HIP_CHECK(hipGetLastError());
         if (evs) FTL_HIP_CHECK(hipEventRecord(evs[1], st));
         hipLaunchKernelGGL(k_eigen_modes<BS>, dim3(a.m), dim3(BS), lds, st, a);
+        FTL_HIP_CHECK(hipGetLastError());
+        if (evs) FTL_HIP_CHECK(hipEventRecord(evs[2], st));
+    }
+
+    // computeM of n draws with `modes_n` sampled modes altogether.
+    void launch_cm_split(const ComputeMSel& sel, uint32_t n, uint32_t modes_n, hipStream_t st, hipEvent_t* evs) {
+        const size_t lds = jacobi_solve_lds_doubles(R) * sizeof(double);
+        const uint32_t bs = jacobi_threads();
+        auto solve = [&](uint32_t blocks, int gram) {
+            auto go = [&](auto bsc, auto two) {
+                constexpr int BS = decltype(bsc)::value;
+                hipLaunchKernelGGL((k_cm_solve<BS, decltype(two)::value>), dim3(blocks), dim3(BS), lds, st, sel, gram);
+            };
+            auto go_bs = [&](auto two) {
+                if (bs == 256) go(std::integral_constant<int, 256>{}, two);
+                else if (bs == 512) go(std::integral_constant<int, 512>{}, two);
+                else go(std::integral_constant<int, 1024>{}, two);
+            };
+            if (R <= (uint64_t)kJacobiDoubleR) go_bs(std::true_type{});
+            else go_bs(std::false_type{});
+            FTL_HIP_CHECK(hipGetLastError());
+            if (R <= 64)
+                hipLaunchKernelGGL(k_cm_vectors<32>, dim3((unsigned)((R + 1) / 2), blocks), dim3(64), 0, st, sel, gram);
+            else
+                hipLaunchKernelGGL(k_cm_vectors<64>, dim3((unsigned)R, blocks), dim3(64), 0, st, sel, gram);
+            FTL_HIP_CHECK(hipGetLastError());
+        };
+        if (evs) FTL_HIP_CHECK(hipEventRecord(evs[0], st));
+        solve(n, 1);
+        hipLaunchKernelGGL(k_cm_pinv, dim3((unsigned)((R * R + 255) / 256), n), dim3(256), 0, st, sel);
+        FTL_HIP_CHECK(hipGetLastError());
+        if (evs) FTL_HIP_CHECK(hipEventRecord(evs[1], st));
+        if (modes_n > n) solve(sel.many ? modes_n : modes_n - 1, 0);
+        hipLaunchKernelGGL(k_cm_etree, dim3((ts64 + 63) / 64, modes_n), dim3(64),
+                           (size_t)etree_nodes * 64 * sizeof(double), st, sel);
         FTL_HIP_CHECK(hipGetLastError());
         if (evs) FTL_HIP_CHECK(hipEventRecord(evs[2], st));
     }
@@ -1556,9 +1611,8 @@ void sampler_draw_packed(const PackItem* items, uint32_t n, void* dev_args, void
     FTL_HIP_CHECK(hipMemcpyAsync(dv, hs, L.total, hipMemcpyHostToDevice, st));
     const ComputeMArgs* cm_dev = (const ComputeMArgs*)(dv + L.cm);
     const uint64_t R = s0->R;
-    const uint64_t jac = 3 * (R + 1) * R <= (uint64_t)kJacobiLdsDoubles ? 3 * (R + 1) * R : (R + 1) * R;
-    const size_t lds = jac * sizeof(double);
-    const uint32_t bs = s0->jacobi_override ? s0->jacobi_override : jacobi_threads_for(R);
+    const uint32_t bs = s0->jacobi_threads();
+    const size_t lds = jacobi_lds_doubles(R) * sizeof(double);
     auto cm_launch = [&](auto bsc) {
         constexpr int BS = decltype(bsc)::value;
         hipLaunchKernelGGL(k_gram_pinv_batched<BS>, dim3(n), dim3(BS), lds, st, cm_dev);
@@ -1567,9 +1621,19 @@ void sampler_draw_packed(const PackItem* items, uint32_t n, void* dev_args, void
                            (const uint32_t*)(dv + L.breq), (const uint32_t*)(dv + L.bpos));
         FTL_HIP_CHECK(hipGetLastError());
     };
-    if (bs == 256) cm_launch(std::integral_constant<int, 256>{});
-    else if (bs == 512) cm_launch(std::integral_constant<int, 512>{});
-    else cm_launch(std::integral_constant<int, 1024>{});
+    if (R >= (uint64_t)kJacobiSplitR) {
+        ComputeMSel sel{};
+        sel.many = cm_dev;
+        sel.req = (const uint32_t*)(dv + L.breq);
+        sel.pos = (const uint32_t*)(dv + L.bpos);
+        items[0].s->launch_cm_split(sel, n, blocks, st, nullptr);
+    } else if (bs == 256) {
+        cm_launch(std::integral_constant<int, 256>{});
+    } else if (bs == 512) {
+        cm_launch(std::integral_constant<int, 512>{});
+    } else {
+        cm_launch(std::integral_constant<int, 1024>{});
+    }
     s0->with_cfg([&](auto rmax, auto sgc) {
         constexpr int RM = decltype(rmax)::value, SG = decltype(sgc)::value, BS = 256;
         const uint64_t blocks_d = std::max<uint64_t>(1, std::min<uint64_t>((off[n] + BS / 64 - 1) / (BS / 64), 1u << 20));

@@ -613,8 +613,11 @@ struct ComputeMArgs {
     double* W;       // R x R, columns = eigvecs / sqrt(lambda), descending lambda
     double* E;       // N x R x R
     double* etree;   // N x etree_nodes x ts64
-    double* work;    // per block: 3 (R+1) R doubles (V and eigenvectors when they do not fit LDS)
-    double* lam_out; // (m+1) x R eigenvalues (diagnostics)
+    double* lam_out; // (m+1) x R eigenvalues
+    // R >= kJacobiSplitR: per solve (the Gram's, then the sampled modes') its
+    // log of rotations, the places of its eigenvalues and its round count
+    double2* log;    // (m+1) x jacobi_log_doubles(R) / 2
+    int* rank;       // (m+1) x (R+1), the count last
     uint32_t ts64;
     uint32_t etree_nodes;
 };
@@ -634,28 +637,31 @@ __device__ inline void fill_pair_table(uint8_t* pa, uint8_t* pb, int R) {
     }
 }
 
+// G = Hadamard product of the sampled root Grams, multiplied in the
+// reference's suffix order G_{m-1} (.) ... (.) G_0 (efficient_krp_sampler.hpp:95-105)
+__device__ inline double cm_gram_entry(const ComputeMArgs& a, int r, int c) {
+    double g = 1.0;
+    for (int t = a.m - 1; t >= 0; t--) g = packed_get(a.roots[a.modes[t]], a.R, r, c) * g;
+    return g;
+}
+
+// P_k = (G_{modes[t+1]} (.) (... (.) G_{modes[m-1]})) (.) pinv
+__device__ inline double cm_mode_entry(const ComputeMArgs& a, int t, int r, int c) {
+    double g = 1.0;
+    for (int s = a.m - 1; s > t; s--) g = packed_get(a.roots[a.modes[s]], a.R, r, c) * g;
+    return g * a.pinv[r * a.R + c];
+}
+
 template <int BS>
 __device__ __forceinline__ void gram_pinv_body(const ComputeMArgs& a, double* smem, JacobiShared& js,
                                                double* diag_tmp) {
 #pragma clang fp contract(off)
     const int R = a.R, R2 = R * R;
-    const int LD = R + 1;
-    const JacobiStore st = jacobi_store(smem, a.work, R);
-    double* A = st.A;
+    const JacobiStore st = jacobi_store_small(smem, R);
     double* lam = a.lam_out;
-    // G = Hadamard product of the sampled root Grams, multiplied in the
-    // reference's suffix order G_{m-1} (.) ... (.) G_0 (efficient_krp_sampler.hpp:95-105);
-    // each pass issues its loads for all entries of the thread at once.
-    for (int e = threadIdx.x; e < R2; e += BS) A[(e / R) * LD + e % R] = 1.0;
-    for (int t = a.m - 1; t >= 0; t--) {
-        const double* G = a.roots[a.modes[t]];
-        for (int e = threadIdx.x; e < R2; e += BS) {
-            const int r = e / R, c = e % R;
-            A[r * LD + c] = packed_get(G, R, r, c) * A[r * LD + c];
-        }
-    }
+    jacobi_fill<BS>(st.A, R, [&](int r, int c) { return cm_gram_entry(a, r, c); });
     __syncthreads();
-    jacobi_block<BS>(A, st.V, R, lam, st.vecs, js, diag_tmp);
+    jacobi_small<BS>(st.A, st.A1, st.V, R, lam, st.vecs, js, diag_tmp);
     const double* vecs = st.vecs;
     // W[u][R-1-v] = V[u][v] / sqrt(lam[v]) when lam[v] > 1e-8 (126-138); W is
     // staged in the (now free) V buffer and copied out for the last mode's E.
@@ -701,29 +707,15 @@ __device__ __forceinline__ void eigen_modes_body(const ComputeMArgs& a, int t, d
 #pragma clang fp contract(off)
     const int k = a.modes[t];  // t: position in the sampled-mode list
     const int R = a.R, R2 = R * R;
-    const int LD = R + 1;
-    const JacobiStore st = jacobi_store(smem, a.work + (uint64_t)(t + 1) * 3 * LD * R, R);
-    double* A = st.A;
+    const JacobiStore st = jacobi_store_small(smem, R);
     double* E = a.E + (uint64_t)k * R2;
     double* El = st.V;  // E staged next to the Jacobi buffers
     fill_pair_table(pa, pb, R);
     if (t + 1 < a.m) {
         double* lam = a.lam_out + (uint64_t)(t + 1) * R;
-        // P_k = (G_{modes[t+1]} (.) (... (.) G_{modes[m-1]})) (.) pinv
-        for (int e = threadIdx.x; e < R2; e += BS) A[(e / R) * LD + e % R] = 1.0;
-        for (int s = a.m - 1; s > t; s--) {
-            const double* G = a.roots[a.modes[s]];
-            for (int e = threadIdx.x; e < R2; e += BS) {
-                const int r = e / R, c = e % R;
-                A[r * LD + c] = packed_get(G, R, r, c) * A[r * LD + c];
-            }
-        }
-        for (int e = threadIdx.x; e < R2; e += BS) {
-            const int r = e / R, c = e % R;
-            A[r * LD + c] = A[r * LD + c] * a.pinv[e];
-        }
+        jacobi_fill<BS>(st.A, R, [&](int r, int c) { return cm_mode_entry(a, t, r, c); });
         __syncthreads();
-        jacobi_block<BS>(A, st.V, R, lam, st.vecs, js, diag_tmp);
+        jacobi_small<BS>(st.A, st.A1, st.V, R, lam, st.vecs, js, diag_tmp);
         const double* vecs = st.vecs;
         for (int e = threadIdx.x; e < R2; e += BS) {
             const int r = e / R, u = e % R;
@@ -779,7 +771,7 @@ __global__ void __launch_bounds__(BS) k_eigen_modes(ComputeMArgs a) {
     extern __shared__ double smem[];
     __shared__ JacobiShared js;
     __shared__ double diag_tmp[128];
-    __shared__ uint8_t pa[8256], pb[8256];
+    __shared__ uint8_t pa[528], pb[528];  // R < kJacobiSplitR
     eigen_modes_body<BS>(a, (int)blockIdx.x, smem, js, diag_tmp, pa, pb);
 }
 
@@ -792,8 +784,118 @@ __global__ void __launch_bounds__(BS) k_eigen_modes_batched(const ComputeMArgs* 
     extern __shared__ double smem[];
     __shared__ JacobiShared js;
     __shared__ double diag_tmp[128];
-    __shared__ uint8_t pa[8256], pb[8256];
+    __shared__ uint8_t pa[528], pb[528];  // R < kJacobiSplitR
     eigen_modes_body<BS>(args[blk_req[blockIdx.x]], (int)blk_pos[blockIdx.x], smem, js, diag_tmp, pa, pb);
+}
+
+// ---------------------------------------------------------------------------
+// computeM over several launches (R >= kJacobiSplitR), for one draw (args `one`)
+// or several of the same R (many: draw b of the Gram launches, (req[b], pos[b])
+// of the mode launches).  The same results as the one-block kernels:
+//   k_cm_solve     diagonalises G / P_k, one block each
+//   k_cm_vectors   the eigenvectors, a row per wave (or half wave): W / E_k
+//   k_cm_pinv      pinv = W W^T; E of the last sampled mode
+//   k_cm_etree     eigen trees, an entry per thread
+// ---------------------------------------------------------------------------
+struct ComputeMSel {
+    ComputeMArgs one;
+    const ComputeMArgs* many;  // or null
+    const uint32_t *req, *pos;
+};
+
+__device__ inline const ComputeMArgs& cm_sel(const ComputeMSel& s, bool gram, uint32_t b, int& t) {
+    t = gram ? -1 : (int)(s.many ? s.pos[b] : b);
+    return s.many ? s.many[gram ? b : s.req[b]] : s.one;
+}
+
+template <int BS, bool TWO>
+__global__ void __launch_bounds__(BS) k_cm_solve(ComputeMSel sel, int gram) {
+#pragma clang fp contract(off)
+    extern __shared__ double smem[];
+    __shared__ JacobiShared js;
+    __shared__ double diag_tmp[128];
+    int t;
+    const ComputeMArgs& a = cm_sel(sel, gram, blockIdx.x, t);
+    if (t + 1 == a.m) return;  // the last mode's E comes from W
+    const int R = a.R, n2 = jacobi_n2(R), LD = n2 + 1;
+    if (gram) jacobi_fill<BS>(smem, R, n2, LD, [&](int r, int c) { return cm_gram_entry(a, r, c); });
+    else jacobi_fill<BS>(smem, R, n2, LD, [&](int r, int c) { return cm_mode_entry(a, t, r, c); });
+    __syncthreads();
+    int* rank = a.rank + (uint64_t)(t + 1) * (R + 1);
+    double* lam = a.lam_out + (uint64_t)(t + 1) * R;
+    double2* log = a.log + (uint64_t)(t + 1) * (jacobi_log_doubles(R) / 2);
+    jacobi_solve<BS, TWO>(smem, smem + n2 * LD, R, log, lam, rank, rank + R, js, diag_tmp);
+}
+
+template <int LPR>
+__global__ void __launch_bounds__(64) k_cm_vectors(ComputeMSel sel, int gram) {
+#pragma clang fp contract(off)
+    int t;
+    const ComputeMArgs& a = cm_sel(sel, gram, blockIdx.y, t);
+    if (t + 1 == a.m) return;
+    const int R = a.R, R2 = R * R;
+    const int i = (int)(blockIdx.x * (64 / LPR) + threadIdx.x / LPR);
+    const double* lam = a.lam_out + (uint64_t)(t + 1) * R;
+    const int* rank = a.rank + (uint64_t)(t + 1) * (R + 1);
+    jacobi_row<LPR>(a.log + (uint64_t)(t + 1) * (jacobi_log_doubles(R) / 2), rank[R], R, i, threadIdx.x,
+                    [&](int v, double x) {
+                        if (i >= R) return;
+                        const int at = rank[v];
+                        const double l = lam[at];
+                        // W[u][R-1-v] = V[u][v] / sqrt(lam[v]) when lam[v] > 1e-8
+                        // (efficient_krp_sampler.hpp:126-138); E rows sqrt(mu) v,
+                        // clamped at 0
+                        if (gram) a.W[i * R + (R - 1 - at)] = l > 1e-8 ? x / sqrt(l) : 0.0;
+                        else a.E[(uint64_t)a.modes[t] * R2 + at * R + i] = x * sqrt(l > 0.0 ? l : 0.0);
+                    });
+}
+
+__global__ void __launch_bounds__(256) k_cm_pinv(ComputeMSel sel) {
+#pragma clang fp contract(off)
+    int t;
+    const ComputeMArgs& a = cm_sel(sel, true, blockIdx.y, t);
+    const int R = a.R, e = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (e >= R * R) return;
+    const int r = e / R, c = e - r * R;
+    const double* wl = a.W + min(r, c) * R;
+    const double* wh = a.W + max(r, c) * R;
+    double acc = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < R; k++) acc = acc + wl[k] * wh[k];
+    a.pinv[e] = acc;
+    a.E[(uint64_t)a.modes[a.m - 1] * R * R + e] = a.W[c * R + r];
+}
+
+// Dynamic LDS: (2 R - 1) x 64 doubles.
+__global__ void __launch_bounds__(64) k_cm_etree(ComputeMSel sel) {
+#pragma clang fp contract(off)
+    extern __shared__ double col[];
+    int t;
+    const ComputeMArgs& a = cm_sel(sel, false, blockIdx.y, t);
+    const int R = a.R, k = a.modes[t];
+    const uint32_t T = (uint32_t)tri_size(R), e = blockIdx.x * 64 + threadIdx.x;
+    if (e >= a.ts64) return;
+    double* v = col + threadIdx.x;
+    // (row, column) of packed entry e
+    int ra = 0, base = 0;
+    while (ra + 1 < R && base + (R - ra) <= (int)e) {
+        base += R - ra;
+        ra++;
+    }
+    const int rb = min(ra + (int)e - base, R - 1);
+    const Shape es = make_shape(R, 1);
+    const uint32_t L = (uint32_t)es.leaf_count, first = (uint32_t)(es.node_count - L);
+    const double* E = a.E + (uint64_t)k * R * R;
+    double* tree = a.etree + (uint64_t)k * a.etree_nodes * a.ts64 + e;
+#pragma unroll 8
+    for (uint32_t i = 0; i < L; i++) {
+        const uint32_t row = (uint32_t)leaf_index(es, first + i);
+        v[(first + i) * 64] = e < T ? E[row * R + ra] * E[row * R + rb] : 0.0;
+    }
+    for (int c = (int)first - 1; c >= 0; c--) v[c * 64] = v[(2 * c + 1) * 64] + v[(2 * c + 2) * 64];
+    const double g = e < T ? a.roots[k][e] : 1.0;
+#pragma unroll 8
+    for (uint32_t c = 0; c < (uint32_t)es.node_count; c++) tree[(uint64_t)c * a.ts64] = v[c * 64] * g;
 }
 
 // ---------------------------------------------------------------------------
