@@ -589,18 +589,45 @@ void pinv_lds_attrs() {
 }
 
 template <int RMAX>
-void launch_gram_rows(const double* X, uint64_t n, uint32_t R, double* parts, unsigned nb, hipStream_t st) {
-    hipLaunchKernelGGL((k_gram_partial<256, RMAX>), dim3(nb), dim3(256), 0, st, X, (const uint32_t*)nullptr, n, R,
-                       parts);
+void launch_gram_rows(const double* X, const uint32_t* n_dev, uint64_t n, uint32_t R, double* parts, unsigned nb,
+                      hipStream_t st) {
+    hipLaunchKernelGGL((k_gram_partial<256, RMAX>), dim3(nb), dim3(256), 0, st, X, n_dev, n, R, parts);
     FTL_LAUNCH_CHECK();
 }
 
-void gram_rows(const double* X, uint64_t n, uint32_t R, double* parts, unsigned nb, hipStream_t st) {
-    if (R <= 8) launch_gram_rows<8>(X, n, R, parts, nb, st);
-    else if (R <= 16) launch_gram_rows<16>(X, n, R, parts, nb, st);
-    else if (R <= 32) launch_gram_rows<32>(X, n, R, parts, nb, st);
-    else if (R <= 64) launch_gram_rows<64>(X, n, R, parts, nb, st);
-    else launch_gram_rows<128>(X, n, R, parts, nb, st);
+template <int NB>
+void launch_gram_mfma(const double* X, const uint32_t* n_dev, uint64_t n, uint32_t R, double* parts, unsigned nb,
+                      hipStream_t st) {
+    hipLaunchKernelGGL(k_gram_mfma<NB>, dim3(nb), dim3(256), 0, st, X, n_dev, n, R, parts);
+    FTL_LAUNCH_CHECK();
+}
+
+// Block partials (nb blocks) of the packed Gram of n rows of X (n from *n_dev
+// when given): on the FP64 matrix cores up to R = 64.
+void gram_rows(const double* X, const uint32_t* n_dev, uint64_t n, uint32_t R, double* parts, unsigned nb,
+               hipStream_t st) {
+    if (R <= 16) launch_gram_mfma<1>(X, n_dev, n, R, parts, nb, st);
+    else if (R <= 32) launch_gram_mfma<2>(X, n_dev, n, R, parts, nb, st);
+    else if (R <= 48) launch_gram_mfma<3>(X, n_dev, n, R, parts, nb, st);
+    else if (R <= 64) launch_gram_mfma<4>(X, n_dev, n, R, parts, nb, st);
+    else launch_gram_rows<128>(X, n_dev, n, R, parts, nb, st);
+}
+
+// Scratch of the allocation-free residual, and its Gram partials' share of it.
+constexpr uint64_t kNoAllocScratchDoubles = 9ull << 17;  // 1,179,648 doubles = 9 MiB
+
+// Blocks of a factor Gram of up to imax rows: 256 rows a block (16 blocks for
+// 65,536 rows left most of the chip idle: 161 us at R = 25), or as many as the
+// allocation-free residual's scratch holds, which sums the same partials; at
+// least the 4,096-row blocks that its size limit is stated in.
+unsigned factor_gram_blocks_min(uint64_t imax) {
+    return (unsigned)std::min<uint64_t>(kGramBlocksMax, std::max<uint64_t>(1, (imax + 4095) / 4096));
+}
+unsigned factor_gram_blocks(uint64_t imax, uint32_t N, uint64_t T) {
+    const uint64_t want = std::min<uint64_t>(kGramBlocksMax, (imax + 255) / 256);
+    const uint64_t held = (kNoAllocScratchDoubles - 4 - kResidBlocks) / T;
+    const uint64_t fit = held > N ? held - N : 0;
+    return std::max(factor_gram_blocks_min(imax), (unsigned)std::min(want, fit));
 }
 
 // rows of the hybrid sampler's candidate lists: lev[i] >= *cut
@@ -741,17 +768,7 @@ struct LKSampler {
         const uint64_t n = I[k];
         const uint32_t r = (uint32_t)R;
         const unsigned nb = (unsigned)std::min<uint64_t>(kGramBlocksMax, std::max<uint64_t>(1, (n + 4095) / 4096));
-        if (r <= 16)
-            hipLaunchKernelGGL(k_gram_mfma<1>, dim3(nb), dim3(256), 0, stream, U[k], n, r, gparts);
-        else if (r <= 32)
-            hipLaunchKernelGGL(k_gram_mfma<2>, dim3(nb), dim3(256), 0, stream, U[k], n, r, gparts);
-        else if (r <= 48)
-            hipLaunchKernelGGL(k_gram_mfma<3>, dim3(nb), dim3(256), 0, stream, U[k], n, r, gparts);
-        else if (r <= 64)
-            hipLaunchKernelGGL(k_gram_mfma<4>, dim3(nb), dim3(256), 0, stream, U[k], n, r, gparts);
-        else
-            gram_rows(U[k], n, r, gparts, nb, stream);
-        FTL_LAUNCH_CHECK();
+        gram_rows(U[k], nullptr, n, r, gparts, nb, stream);
         hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, stream, counters + kCntUnique,
                            (uint32_t)std::min<uint64_t>(n, R));
         FTL_LAUNCH_CHECK();
@@ -1116,20 +1133,8 @@ struct Als {
         FTL_HIP_CHECK(hipEventRecord(ev[i], stream));
     }
 
-    template <int RMAX>
-    void launch_gram(const double* Xrows, const uint32_t* n_dev, uint64_t n_host, double* parts, unsigned nb) {
-        hipLaunchKernelGGL((k_gram_partial<256, RMAX>), dim3(nb), dim3(256), 0, stream, Xrows, n_dev, n_host,
-                           (uint32_t)R, parts);
-        FTL_LAUNCH_CHECK();
-    }
-
-    // block partials (nb blocks) of the packed Gram of n rows
     void gram_partials(const double* Xrows, const uint32_t* n_dev, uint64_t n_host, double* parts, unsigned nb) {
-        if (R <= 8) launch_gram<8>(Xrows, n_dev, n_host, parts, nb);
-        else if (R <= 16) launch_gram<16>(Xrows, n_dev, n_host, parts, nb);
-        else if (R <= 32) launch_gram<32>(Xrows, n_dev, n_host, parts, nb);
-        else if (R <= 64) launch_gram<64>(Xrows, n_dev, n_host, parts, nb);
-        else launch_gram<128>(Xrows, n_dev, n_host, parts, nb);
+        gram_rows(Xrows, n_dev, n_host, (uint32_t)R, parts, nb, stream);
     }
 
     // The last sampled update's draw: samples (N x J, the excluded mode's row
@@ -1216,7 +1221,7 @@ struct Als {
         if (renormalize) {
             if (T > 0) {
                 // column sums of squares of the touched rows came with the row finalise
-                hipLaunchKernelGGL(k_colnorm_final, dim3(1), dim3(256), 0, st, colpart, colparts, (uint32_t)R, norms,
+                hipLaunchKernelGGL(k_colnorm_final, dim3((unsigned)R), dim3(256), 0, st, colpart, colparts, (uint32_t)R, norms,
                                    sigma, 0);
                 FTL_LAUNCH_CHECK();
                 hipLaunchKernelGGL(k_scale_rows, dim3(grid_for(T * R, 256)), dim3(256), 0, st, U[j], mt.seg_row,
@@ -1302,7 +1307,7 @@ struct Als {
         else if (R <= 64) parts = launch_exact<64, 1>(o, j, colsq);
         else parts = launch_exact<64, 2>(o, j, colsq);
         if (renormalize) {
-            hipLaunchKernelGGL(k_colnorm_final, dim3(1), dim3(256), 0, st, colpart, parts, (uint32_t)R, norms, sigma, 0);
+            hipLaunchKernelGGL(k_colnorm_final, dim3((unsigned)R), dim3(256), 0, st, colpart, parts, (uint32_t)R, norms, sigma, 0);
             FTL_LAUNCH_CHECK();
             hipLaunchKernelGGL(k_scale_rows, dim3(grid_for(o.D * R, 256)), dim3(256), 0, st, U[j], o.seg_row,
                                o.counters + kCntRows, (uint64_t)0, (uint32_t)R, norms);
@@ -1326,7 +1331,7 @@ struct Als {
             hipLaunchKernelGGL(k_colsq_partial<256>, dim3(kColBlocks), dim3(256), 0, st, U[k], nullptr, nullptr, I[k],
                                (uint32_t)R, colpart);
             FTL_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_colnorm_final, dim3(1), dim3(256), 0, st, colpart, kColBlocks, (uint32_t)R, norms,
+            hipLaunchKernelGGL(k_colnorm_final, dim3((unsigned)R), dim3(256), 0, st, colpart, kColBlocks, (uint32_t)R, norms,
                                sigma, j == -1 ? 1 : 0);
             FTL_LAUNCH_CHECK();
             hipLaunchKernelGGL(k_scale_rows, dim3(grid_for(I[k] * R, 256)), dim3(256), 0, st, U[k], nullptr, nullptr,
@@ -1341,9 +1346,9 @@ struct Als {
         const uint64_t T = R * (R + 1) / 2;
         uint64_t imax = 1;
         for (uint32_t k = 0; k < N; k++) imax = std::max(imax, I[k]);
-        const unsigned nb = (unsigned)std::min<uint64_t>(kGramBlocksMax, std::max<uint64_t>(1, (imax + 4095) / 4096));
+        const unsigned nb = factor_gram_blocks(imax, N, T);
         for (uint32_t k = 0; k < N; k++) gram_partials(U[k], nullptr, I[k], gram_parts + (uint64_t)k * nb * T, nb);
-        hipLaunchKernelGGL(k_gram_reduce, dim3(grid_for(N * T, 256)), dim3(256), 0, stream, gram_parts, nb,
+        hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)((8 * N * T + 255) / 256)), dim3(256), 0, stream, gram_parts, nb,
                            (uint32_t)T, N, gram_red);
         FTL_LAUNCH_CHECK();
     }
@@ -1433,8 +1438,6 @@ uint64_t jacobi_capped_als_tu() { return jacobi_capped_read(); }
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr uint64_t kNoAllocScratchDoubles = 9ull << 17;  // 1,179,648 doubles = 9 MiB
-
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];
 
 std::mutex g_scratch_mu;
@@ -1459,13 +1462,6 @@ __global__ void k_add_pair(const double* __restrict__ two, double* __restrict__ 
     if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = two[0] + two[1];
 }
 
-template <int RMAX>
-void noalloc_gram(const double* U, uint64_t n, uint32_t R, double* parts, unsigned nb, hipStream_t st) {
-    hipLaunchKernelGGL((k_gram_partial<256, RMAX>), dim3(nb), dim3(256), 0, st, U, (const uint32_t*)nullptr, n, R,
-                       parts);
-    FTL_LAUNCH_CHECK();
-}
-
 }  // namespace
 
 // The same kernels, in the same order and with the same grids, as
@@ -1483,9 +1479,9 @@ void residual_normsq_noalloc(SparseDev& X, uint64_t R, const uint64_t* I, const 
         FTL_REQUIRE(I[k] >= X.dims[k], "factor has fewer rows than the tensor's mode size");
         imax = std::max(imax, I[k]);
     }
-    const unsigned nb = (unsigned)std::min<uint64_t>(kGramBlocksMax, std::max<uint64_t>(1, (imax + 4095) / 4096));
+    const unsigned nb_min = factor_gram_blocks_min(imax), nb = factor_gram_blocks(imax, N, T);
     // layout: [scal 4][resid_part kResidBlocks][gram_red N T][gram_parts nb T]
-    const uint64_t need = 4 + kResidBlocks + (uint64_t)N * T + (uint64_t)nb * T;
+    const uint64_t need = 4 + kResidBlocks + (uint64_t)N * T + (uint64_t)nb_min * T;
     if (need > kNoAllocScratchDoubles)
         throw Error{FTL_EUNSUPPORTED, "the residual needs " + std::to_string(need * 8) + " bytes of scratch for R = " +
                                           std::to_string(R) + " and " + std::to_string(imax) +
@@ -1515,12 +1511,8 @@ void residual_normsq_noalloc(SparseDev& X, uint64_t R, const uint64_t* I, const 
     hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, st, resid_part, kResidBlocks, scal);
     FTL_LAUNCH_CHECK();
     for (uint32_t k = 0; k < N; k++) {
-        if (R <= 8) noalloc_gram<8>(U[k], I[k], Ru, gram_parts, nb, st);
-        else if (R <= 16) noalloc_gram<16>(U[k], I[k], Ru, gram_parts, nb, st);
-        else if (R <= 32) noalloc_gram<32>(U[k], I[k], Ru, gram_parts, nb, st);
-        else if (R <= 64) noalloc_gram<64>(U[k], I[k], Ru, gram_parts, nb, st);
-        else noalloc_gram<128>(U[k], I[k], Ru, gram_parts, nb, st);
-        hipLaunchKernelGGL(k_gram_reduce, dim3(grid_for(T, 256)), dim3(256), 0, st, gram_parts, nb, (uint32_t)T, 1u,
+        gram_rows(U[k], nullptr, I[k], Ru, gram_parts, nb, st);
+        hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)((8 * T + 255) / 256)), dim3(256), 0, st, gram_parts, nb, (uint32_t)T, 1u,
                            gram_red + (uint64_t)k * T);
         FTL_LAUNCH_CHECK();
     }

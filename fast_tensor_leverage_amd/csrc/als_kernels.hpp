@@ -319,6 +319,10 @@ __device__ bool pinv_cholesky(const double* A, double* C, double* Li, int R, dou
     }
     if (tid == 0) fail = 0;
     __syncthreads();
+    // step k: row k of L^-1 (lower; x_j = 1 / l_jj, x_i = -(sum_{m=j}^{i-1} l_im
+    // x_m) / l_ii, the sums running in Li), column k of L, then the trailing
+    // update of both.  (The inverse a column per thread after the factor was a
+    // chain of R^2 / 2 dependent steps, half of this kernel's 44 us at R = 25.)
     for (int k = 0; k < R; k++) {
         const double piv = C[k * LD + k];
         __syncthreads();
@@ -326,25 +330,18 @@ __device__ bool pinv_cholesky(const double* A, double* C, double* Li, int R, dou
         const double lkk = sqrt(piv);
         for (int i = k + 1 + tid; i < R; i += BS) C[i * LD + k] = C[i * LD + k] / lkk;
         if (tid == 0) C[k * LD + k] = lkk;
+        // the row on the block's last waves, beside the column
+        for (int j = BS - 1 - tid; j < R; j += BS)
+            Li[k * R + j] = j < k ? (0.0 - Li[k * R + j]) / lkk : j == k ? 1.0 / lkk : 0.0;
         __syncthreads();
-        const int m = R - k - 1;  // trailing block, lower triangle
-        for (int e = tid; e < m * m; e += BS) {
-            const int i = k + 1 + e / m, j = k + 1 + e % m;
-            if (j <= i) C[i * LD + j] = C[i * LD + j] - C[i * LD + k] * C[j * LD + k];
+        const int m = R - k - 1;  // trailing rows
+        for (int e = tid; e < m * R; e += BS) {
+            const int i = k + 1 + e / R, j = e % R;
+            if (j > k && j <= i) C[i * LD + j] = C[i * LD + j] - C[i * LD + k] * C[j * LD + k];
+            if (j <= k) Li[i * R + j] = (j == k ? 0.0 : Li[i * R + j]) + C[i * LD + k] * Li[k * R + j];
         }
         __syncthreads();
     }
-    // column j of L^-1 (lower): x_j = 1 / l_jj, x_i = -(sum_{m=j}^{i-1} l_im x_m) / l_ii
-    for (int j = tid; j < R; j += BS) {
-        for (int i = 0; i < j; i++) Li[i * R + j] = 0.0;
-        Li[j * R + j] = 1.0 / C[j * LD + j];
-        for (int i = j + 1; i < R; i++) {
-            double s = 0.0;
-            for (int m = j; m < i; m++) s = s + C[i * LD + m] * Li[m * R + j];
-            Li[i * R + j] = (0.0 - s) / C[i * LD + i];
-        }
-    }
-    __syncthreads();
     // A^-1 = Li^T Li into pinv; Frobenius norms of A^-1 and A
     double f_inv = 0.0, f_a = 0.0;
     for (int e = tid; e < R * R; e += BS) {
@@ -1072,24 +1069,30 @@ __global__ void __launch_bounds__(BS) k_colsq_partial(const double* __restrict__
 }
 
 // norms[c] = sqrt(sum of the partials), 1 when <= 1e-7; sigma either the
-// norms or sigma * norms (multiply).  One block of 256 threads: wave w sums
-// columns w, w+4, ...; lane l adds partials l, l+64, ... in order, then a
-// fixed xor butterfly over the 64 lanes.
+// norms or sigma * norms (multiply).  A block of 256 threads per column: thread t
+// adds partials t, t + 256, ... in order, then a fixed tree over the threads.
+// (One block for all columns took 37-47 us for R = 25 and 2,048 partials, a chain
+// of 224 dependent loads per wave; this takes 5.)
 __global__ void __launch_bounds__(256) k_colnorm_final(const double* __restrict__ partial, uint32_t nparts,
                                                        uint32_t R, double* __restrict__ norms,
                                                        double* __restrict__ sigma, int multiply) {
 #pragma clang fp contract(off)
-    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (uint32_t c = wv; c < R; c += 4) {
-        double s = 0.0;
-        for (uint32_t p = lane; p < nparts; p += 64) s += partial[(uint64_t)p * R + c];
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        if (lane == 0) {
-            double nrm = sqrt(s);
-            if (nrm <= 1e-7) nrm = 1.0;
-            norms[c] = nrm;
-            if (sigma) sigma[c] = multiply ? sigma[c] * nrm : nrm;
-        }
+    __shared__ double red[256];
+    const uint32_t c = blockIdx.x;
+    double s = 0.0;
+#pragma unroll 8
+    for (uint32_t p = threadIdx.x; p < nparts; p += 256) s += partial[(uint64_t)p * R + c];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (uint32_t h = 128; h > 0; h >>= 1) {
+        if (threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        double nrm = sqrt(red[0]);
+        if (nrm <= 1e-7) nrm = 1.0;
+        norms[c] = nrm;
+        if (sigma) sigma[c] = multiply ? sigma[c] * nrm : nrm;
     }
 }
 
@@ -1196,19 +1199,24 @@ __global__ void __launch_bounds__(BS) k_residual_partial(const uint64_t* __restr
     }
 }
 
-// Sum of nparts block partials of packed Grams, per entry (grid over
-// nmodes x T entries; each thread adds its entry's partials in order).
-__global__ void k_gram_reduce(const double* __restrict__ parts, uint32_t nparts, uint32_t T, uint32_t nmodes,
-                              double* __restrict__ out) {
+// Sum of nparts block partials of packed Grams, per entry (nmodes x T entries,
+// eight lanes each): lane h adds the partials [h c, (h+1) c), c = ceil(nparts /
+// 8), in order, and the eight sums are added in order.
+__global__ void __launch_bounds__(256) k_gram_reduce(const double* __restrict__ parts, uint32_t nparts, uint32_t T,
+                                                     uint32_t nmodes, double* __restrict__ out) {
 #pragma clang fp contract(off)
-    const uint64_t n = (uint64_t)nmodes * T;
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < n; w += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t k = w / T, e = w - k * T;
-        const double* P = parts + k * nparts * T;
-        double s = 0.0;
-        for (uint32_t p = 0; p < nparts; p++) s += P[(uint64_t)p * T + e];
-        out[w] = s;
-    }
+    const uint64_t idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint64_t w = min<uint64_t>(idx >> 3, (uint64_t)nmodes * T - 1), k = w / T, e = w - k * T;
+    const uint32_t h = (uint32_t)idx & 7, c = (nparts + 7) / 8;
+    const uint32_t pb = min(nparts, h * c), pe = min(nparts, pb + c);
+    const double* P = parts + k * nparts * T + e;
+    double s = 0.0;
+#pragma unroll 16
+    for (uint32_t p = pb; p < pe; p++) s += P[(uint64_t)p * T];
+    double t = 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; u++) t += __shfl(s, u, 8);
+    if (h == 0 && (idx >> 3) < (uint64_t)nmodes * T) out[w] = t;
 }
 
 // ||M||^2 = sum_{a,b} sigma_a sigma_b prod_k G_k[a][b] (common.h:152-226) from
@@ -1264,12 +1272,13 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 // wave order.  partial[b0] holds the packed upper triangle (entry (r, c),
 // r <= c, at r R - r(r-1)/2 + c - r), the layout k_pinv_partials reduces.
 template <int NB>
-__global__ void __launch_bounds__(256) k_gram_mfma(const double* __restrict__ U, uint64_t I, uint32_t R,
-                                                   double* __restrict__ partial) {
+__global__ void __launch_bounds__(256) k_gram_mfma(const double* __restrict__ U, const uint32_t* n_dev,
+                                                   uint64_t n_host, uint32_t R, double* __restrict__ partial) {
     constexpr int NT = NB * (NB + 1) / 2;
     constexpr int UNR = NB <= 2 ? 8 : 4;  // 16-row steps per loop trip (loads in flight)
     __shared__ double red[4][4][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t I = n_dev ? (uint64_t)*n_dev : n_host;
     const uint64_t chunk = (((I + gridDim.x - 1) / gridDim.x) + 15) & ~15ull;
     const uint64_t rb = (uint64_t)blockIdx.x * chunk;
     const uint64_t re = min<uint64_t>(I, rb + chunk);
