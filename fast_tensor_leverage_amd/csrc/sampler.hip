@@ -620,13 +620,15 @@ struct Sampler {
 
     // Builds on a stream other than the sampler's own occur only for samplers
     // on a borrowed stream, which keep one computeM set on that stream.
-    void build_mode(uint32_t k, hipStream_t st = nullptr) {
+    // src: the factor to build from (device), copied to U64 on the way; null: U64.
+    void build_mode(uint32_t k, hipStream_t st = nullptr, const double* src = nullptr) {
         if (!st) st = stream;
         if (st == stream) wait_foreign_draws();
         trees_dirty = true;
         ModeHost& m = modes[k];
         BuildArgs ba;
-        ba.U = m.U64;
+        ba.U = src ? src : m.U64;
+        ba.Ucopy = src && src != m.U64 ? m.U64 : nullptr;
         ba.tree = m.tree64;
         ba.sh = m.sh;
         ba.R = (uint32_t)R;
@@ -686,15 +688,25 @@ struct Sampler {
             else
                 hipLaunchKernelGGL(k_leaf_gram_mfma<4>, dim3((unsigned)lblocks), dim3(256), 0, st, ba);
         } else {
-            // leaves per block: their row blocks within 32 KB of LDS (a power
-            // of two <= 8, at least one leaf); entries bitwise the oracle's
-            const uint64_t leaf_doubles = std::max<uint64_t>(1, m.F * R);
-            uint32_t lpb = 1;
-            while (lpb < 8 && 2 * lpb * leaf_doubles <= 4096) lpb *= 2;
-            const size_t lds = (size_t)lpb * leaf_doubles * sizeof(double) + tri_size(R) * sizeof(uint16_t);
-            const uint64_t lblocks = (m.sh.leaf_count + lpb - 1) / lpb;
+            // as many leaves per block as tiles fit 256 threads within 20 KB of
+            // LDS, and at least one; a tile per thread, so up to 1,024 threads
+            // where one leaf has more than 256 tiles (R > 88).  Blocks a CU holds
+            // bound the kernel: a construction over three factors of 2^21 x 32
+            // takes 1,405 / 1,463 / 1,576 us with 20 / 32 / 48 KB, of 2^22 x 8
+            // 824 / 887 / 895.
+            constexpr uint32_t kLeafLdsDoubles = 2560;
+            LeafLayout L;
+            L.rs = (uint32_t)(R + 3) / 4 * 4;
+            L.tiles = (L.rs / 4) * (L.rs / 4 + 1) / 2;
+            const uint32_t maxt = L.tiles <= 256 ? 256u : 1024u;
+            L.stride = (uint32_t)std::max<uint64_t>(m.F * L.rs, ts64) + 16;
+            L.lpb = std::max<uint32_t>(1, std::min<uint32_t>(maxt / L.tiles, kLeafLdsDoubles / L.stride));
+            L.threads = (L.lpb * L.tiles + 63) / 64 * 64;
+            const size_t lds = (size_t)L.lpb * L.stride * sizeof(double);
+            const uint64_t lblocks = (m.sh.leaf_count + L.lpb - 1) / L.lpb;
             FTL_REQUIRE(lblocks <= 0x7fffffffull, "too many leaves for one launch");
-            hipLaunchKernelGGL(k_leaf_gram<256>, dim3((unsigned)lblocks), dim3(256), lds, st, ba, lpb);
+            hipLaunchKernelGGL(maxt == 256 ? k_leaf_gram<256> : k_leaf_gram<1024>, dim3((unsigned)lblocks),
+                               dim3(L.threads), lds, st, ba, L);
         }
         FTL_HIP_CHECK(hipGetLastError());
         // internal nodes of the lfill level (parents of a partial bottom level)
@@ -898,8 +910,8 @@ struct Sampler {
         // once per process (thread-safe: a throw leaves it to the next call)
         static std::once_flag attrs_once;
         std::call_once(attrs_once, [] {
-            FTL_HIP_CHECK(hipFuncSetAttribute((const void*)k_leaf_gram<256>,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            for (const void* f : {(const void*)k_leaf_gram<256>, (const void*)k_leaf_gram<1024>})
+                FTL_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
             const void* sb[] = {(const void*)k_subtree_build<1, 4>,  (const void*)k_subtree_build<2, 4>,
                                 (const void*)k_subtree_build<3, 4>,  (const void*)k_subtree_build<4, 4>,
                                 (const void*)k_subtree_build<1, 8>,  (const void*)k_subtree_build<2, 8>,
@@ -945,12 +957,13 @@ struct Sampler {
                 m.U64 = const_cast<double*>(U[k]);
             } else {
                 m.U64 = dalloc<double>(m.I * R);
-                FTL_HIP_CHECK(hipMemcpyAsync(m.U64, U[k], m.I * R * sizeof(double),
-                                             on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, stream));
+                if (!on_device)
+                    FTL_HIP_CHECK(hipMemcpyAsync(m.U64, U[k], m.I * R * sizeof(double), hipMemcpyHostToDevice,
+                                                 stream));
             }
             alloc_trees(m);
             if (precision == FTL_FP32) m.U32 = dalloc<float>(m.I * R);
-            build_mode(k);
+            build_mode(k, nullptr, on_device && !alias ? U[k] : nullptr);
         }
         const uint64_t R2 = R * R;
         etree_nodes = (uint32_t)(2 * R - 1);
@@ -1037,9 +1050,9 @@ struct Sampler {
         FTL_REQUIRE(Uj != nullptr, "update_sampler: null factor");
         ModeHost& m = modes[j];
         wait_foreign_draws();
-        FTL_HIP_CHECK(hipMemcpyAsync(m.U64, Uj, m.I * R * sizeof(double),
-                                     on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, stream));
-        build_mode(j);
+        if (!on_device)
+            FTL_HIP_CHECK(hipMemcpyAsync(m.U64, Uj, m.I * R * sizeof(double), hipMemcpyHostToDevice, stream));
+        build_mode(j, nullptr, on_device ? Uj : nullptr);
     }
 
     std::vector<int> sampled_modes(uint32_t j) const {

@@ -35,6 +35,7 @@ namespace ftl {
 // ---------------------------------------------------------------------------
 struct BuildArgs {
     const double* U;   // n x R
+    double* Ucopy;     // or null: where the kernels that read U store it too
     double* tree;      // node_count x ts64
     Shape sh;
     uint32_t R;
@@ -55,52 +56,148 @@ __device__ inline void store_f32(float* tree32, uint64_t n64, uint32_t ts32, uin
     if (tree32 && c >= n64) tree32[(c - n64) * ts32 + e] = e < ts64 ? (float)v : 0.0f;
 }
 
-// lpb leaves per block (BS / lpb threads each).  Dynamic LDS: the leaves'
-// row blocks (lpb x F x R doubles), then the (row, column) of every packed
-// entry (T uint16).  Entry e of a leaf is the sequential sum over its rows.
-template <int BS>
-__global__ void __launch_bounds__(BS) k_leaf_gram(BuildArgs a, uint32_t lpb) {
+// Layout of a k_leaf_gram block: rows of `rs` doubles (R rounded up to 4, zero
+// past R) and `tiles` 4 x 4 tiles of the upper triangle per leaf, `lpb` leaves of
+// `stride` doubles of LDS (the rows, then the packed node in their place; the
+// 16 doubles more put neighbouring leaves on other banks), `threads` in the block.
+struct LeafLayout {
+    uint32_t rs, tiles, lpb, stride, threads;
+};
+
+// A thread holds a 4 x 4 tile of a leaf's Gram in registers: eight LDS entries
+// per row for 16 products (an entry per thread needs 32, which bounds it by the
+// LDS), and the tiles of several leaves fill the block.  Each entry is the
+// sequential sum over the leaf's rows.  The rows are read eight loads ahead, the
+// factor's copy is written as they pass, and a node packed in LDS is written in
+// whole lines: now bounded by those three streams.  Constructing a sampler over
+// three device factors, with the levels above (us; an entry per thread after a
+// copy of the factor -> this): 2^22 x 8 1,124 -> 824, 2^21 x 32 2,172 -> 1,405,
+// 2^20 x 64 2,484 -> 1,730, 2^19 x 128 6,622 -> 2,825.
+template <int MAXT>
+__global__ void __launch_bounds__(MAXT) k_leaf_gram(BuildArgs a, LeafLayout L) {
 #pragma clang fp contract(off)
     extern __shared__ double lds_u[];
     const uint32_t R = a.R;
     const uint32_t F = (uint32_t)a.sh.F;
     const uint32_t T = (uint32_t)tri_size(R);
-    uint16_t* pairs = reinterpret_cast<uint16_t*>(lds_u + (uint64_t)lpb * F * R);
-    for (uint32_t r = threadIdx.x; r < R; r += BS) {
-        const uint32_t base = r * R - r * (r - 1) / 2;
-        for (uint32_t c = r; c < R; c++) pairs[base + c - r] = (uint16_t)(r | (c << 8));
+    const uint64_t i0 = (uint64_t)blockIdx.x * L.lpb;
+    const uint32_t leaves = (uint32_t)min<uint64_t>(L.lpb, a.sh.leaf_count - i0);
+    const uint32_t tid = threadIdx.x, nt = L.threads;
+    const uint64_t node0 = a.first_leaf + i0;
+    {
+        // The leaves' rows, which follow one another in U up to the first leaf of
+        // the bottom level (its rows begin at row 0), as one run of elements:
+        // eight loads a thread are issued before the first is stored.
+        const uint32_t leaf = F * R, total = leaves * leaf;
+        const uint64_t limit = a.sh.n * R;
+        const uint64_t base = leaf_index(a.sh, node0) * leaf;
+        const uint32_t turn = node0 < a.sh.nodes_upto_lfill
+                                  ? (uint32_t)min<uint64_t>(a.sh.nodes_upto_lfill - node0, leaves) * leaf
+                                  : total;
+        const double* __restrict__ U = a.U;
+        double* __restrict__ Uc = a.Ucopy;
+        float* __restrict__ U32 = a.U32;
+        const uint32_t dq = nt / leaf, dr = (nt - dq * leaf) / R, dc = nt - dq * leaf - dr * R;
+        uint32_t q = tid / leaf, row = (tid - q * leaf) / R, col = tid - q * leaf - row * R;
+        for (uint32_t e0 = tid; e0 < total; e0 += 8 * nt) {
+            double x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint32_t e = e0 + u * nt;
+                const uint64_t g = e < turn ? base + e : e - turn;
+                x[u] = e < total && g < limit ? U[g] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint32_t e = e0 + u * nt;
+                const uint64_t g = e < turn ? base + e : e - turn;
+                if (e < total) {
+                    lds_u[q * L.stride + row * L.rs + col] = x[u];
+                    if (g < limit) {
+                        if (Uc) Uc[g] = x[u];
+                        if (U32) U32[g] = (float)x[u];
+                    }
+                }
+                col += dc;
+                row += dr;
+                q += dq;
+                if (col >= R) {
+                    col -= R;
+                    row++;
+                }
+                if (row >= F) {
+                    row -= F;
+                    q++;
+                }
+            }
+        }
+        const uint32_t pad = L.rs - R;
+        if (pad)
+            for (uint32_t e = tid; e < leaves * F; e += nt) {
+                const uint32_t p = e / F;
+                double* z = lds_u + p * L.stride + (e - p * F) * L.rs + R;
+                for (uint32_t c = 0; c < pad; c++) z[c] = 0.0;
+            }
     }
-    const uint32_t tpl = BS / lpb;
-    const uint32_t q = threadIdx.x / tpl, lt = threadIdx.x - q * tpl;
-    const uint64_t i = (uint64_t)blockIdx.x * lpb + q;  // leaf position
-    const bool have = q < lpb && i < a.sh.leaf_count;
-    uint64_t node = 0, r0 = 0;
-    uint32_t rows = 0;
-    double* lu = lds_u + (uint64_t)q * F * R;
+    __syncthreads();
+    const uint32_t q = tid / L.tiles, tl = tid - q * L.tiles;
+    const bool have = q < leaves;
+    double acc[4][4];
+    uint32_t ta = 0, tb = tl;  // tile row and column: tl counts the upper triangle row by row
+    double* lu = lds_u + (uint64_t)(have ? q : 0) * L.stride;
     if (have) {
-        node = a.first_leaf + i;
-        r0 = leaf_index(a.sh, node) * F;
-        rows = (uint32_t)min<uint64_t>(F, a.sh.n - r0);
-        const double* src = a.U + r0 * R;
-        for (uint32_t e = lt; e < rows * R; e += tpl) {
-            const double x = src[e];
-            lu[e] = x;
-            if (a.U32) a.U32[r0 * R + e] = (float)x;
+        for (uint32_t len = L.rs / 4; tb >= len; len--) {
+            tb -= len;
+            ta++;
+        }
+        tb += ta;
+        const uint64_t r0 = leaf_index(a.sh, node0 + q) * F;
+        const uint32_t rows = (uint32_t)min<uint64_t>(F, a.sh.n - r0);
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+#pragma unroll
+            for (int y = 0; y < 4; y++) acc[x][y] = 0.0;
+        const double2* pa = reinterpret_cast<const double2*>(lu + 4 * ta);
+        const double2* pb = reinterpret_cast<const double2*>(lu + 4 * tb);
+#pragma unroll 2
+        for (uint32_t t = 0; t < rows; t++) {
+            const double2 a0 = pa[t * (L.rs / 2)], a1 = pa[t * (L.rs / 2) + 1];
+            const double2 b0 = pb[t * (L.rs / 2)], b1 = pb[t * (L.rs / 2) + 1];
+            const double va[4] = {a0.x, a0.y, a1.x, a1.y}, vb[4] = {b0.x, b0.y, b1.x, b1.y};
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+#pragma unroll
+                for (int y = 0; y < 4; y++) acc[x][y] = acc[x][y] + va[x] * vb[y];
+        }
+    }
+    __syncthreads();  // the rows are read
+    if (have) {
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            const uint32_t r = 4 * ta + x;
+            const uint32_t base = r * R - r * (r + 1) / 2;
+#pragma unroll
+            for (int y = 0; y < 4; y++) {
+                const uint32_t c = 4 * tb + y;
+                if (r <= c && c < R) lu[base + c] = acc[x][y];
+            }
         }
     }
     __syncthreads();
-    if (!have) return;
-    double* out = a.tree + node * (uint64_t)a.ts64;
+    // the packed nodes, one run of `tsw` entries each
     const uint32_t tsw = a.tree32 && a.ts32 > a.ts64 ? a.ts32 : a.ts64;
-    for (uint32_t e = lt; e < tsw; e += tpl) {
-        double acc = 0.0;
-        if (e < T) {
-            const uint32_t ab = pairs[e];
-            const uint32_t ra = ab & 0xffu, cb = ab >> 8;
-            for (uint32_t t = 0; t < rows; t++) acc = acc + lu[t * R + ra] * lu[t * R + cb];
+    const uint32_t dp = nt / tsw, de = nt - dp * tsw;
+    uint32_t p = tid / tsw, e = tid - p * tsw;
+    while (p < leaves) {
+        const double v = e < T ? lds_u[p * L.stride + e] : 0.0;
+        if (e < a.ts64) a.tree[(node0 + p) * a.ts64 + e] = v;
+        store_f32(a.tree32, a.n64, a.ts32, a.ts64, node0 + p, e, v);
+        p += dp;
+        e += de;
+        if (e >= tsw) {
+            e -= tsw;
+            p++;
         }
-        if (e < a.ts64) out[e] = acc;
-        store_f32(a.tree32, a.n64, a.ts32, a.ts64, node, e, acc);
     }
 }
 
@@ -130,6 +227,7 @@ __device__ inline void leaf_mfma_tiles(const BuildArgs& a, uint64_t node, uint32
     const uint32_t kr = lane >> 4, ci = lane & 15;
     const double* __restrict__ U = a.U + r0 * R;
     float* __restrict__ U32 = a.U32 ? a.U32 + r0 * R : nullptr;
+    double* __restrict__ Uc = a.Ucopy ? a.Ucopy + r0 * R : nullptr;
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t] = lg_f64x4{0.0, 0.0, 0.0, 0.0};
     // four 4-row steps per trip: their 4 NB loads are issued before the MFMAs
@@ -152,6 +250,17 @@ __device__ inline void leaf_mfma_tiles(const BuildArgs& a, uint64_t node, uint32
                 for (int b = 0; b < NB; b++) {
                     const uint32_t col = 16 * b + ci;
                     if (row < rows && col < R) U32[row * R + col] = (float)x[u][b];
+                }
+            }
+        }
+        if (Uc) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const uint32_t row = s16 + 4 * u + kr;
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const uint32_t col = 16 * b + ci;
+                    if (row < rows && col < R) Uc[row * R + col] = x[u][b];
                 }
             }
         }
