@@ -576,8 +576,8 @@ unsigned reduce_matches(SparseDev& X, uint32_t j, uint64_t n, uint64_t T, const 
 // target rank min(I_k, R), compute_pinv, common.h:271-323), their prefix sums
 // and total; a draw samples every mode k != j independently from them.
 // ---------------------------------------------------------------------------
-// The one-block pinv kernels hold A ((R+1) R doubles) in LDS, plus V and
-// the eigenvectors when R <= 64: allow up to 132 KB of dynamic LDS.
+// The one-block pinv kernels hold A in LDS, with a second copy, V and the
+// rotations when R <= 64 (jacobi_lds_doubles): allow 132 KB, one copy at R = 128.
 void pinv_lds_attrs() {
     static std::once_flag once;  // thread-safe; a throw leaves it to the next call
     std::call_once(once, [] {
@@ -1098,9 +1098,9 @@ struct Als {
             // after an update a factor is zero in all rows without a matched
             // nonzero and dominated by a few heavy ones: most samples descend to
             // nodes that the caches hold anyway, and the others' paths follow
-            // their uniforms less.  Per sweep: ordered 5,700, in tiles 5,699,
-            // plain 5,540-5,609 us at 2^20 x 2^19 x 2^15, 2e7 nonzeros, R = 25;
-            // in tiles 6,417, plain 6,341 at 183 x 24 x 1140 x 1717.
+            // their uniforms less.  Per sweep: ordered 4,706-4,764, in tiles
+            // 4,838-4,853, plain 4,550-4,573 us at 2^20 x 2^19 x 2^15, 2e7
+            // nonzeros, R = 25; in tiles 5,091, plain 4,799 at 183 x 24 x 1140 x 1717.
             sampler_set_option(sampler, "tile_descent", 0);
             sampler_set_option(sampler, "sample_order", 0);
         }

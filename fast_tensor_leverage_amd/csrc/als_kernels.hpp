@@ -300,9 +300,9 @@ __global__ void __launch_bounds__(BS) k_gram_partial(const double* __restrict__ 
 // common.h:228-269): lambda_min(A) >= 1 / ||A^-1||_F > 2e-11 certifies that
 // no eigenvalue would be cut.  Also required: ||A||_F ||A^-1||_F < 1e6, so
 // the result agrees with the eigendecomposition route to rounding.  C (R
-// (R+1) doubles) and Li (R^2) are scratch.  Right-looking Cholesky (a column
-// per step), the inverse of the factor a column per thread (forward
-// substitution), pinv = Li^T Li; every sum in a fixed order.  Returns false
+// (R+1) doubles) and Li (R^2) are scratch.  Right-looking Cholesky and inverse of
+// its factor (a column of one and a row of the other per step), pinv = Li^T Li;
+// every sum in a fixed order.  Returns false
 // (pinv untouched) when a pivot is not positive or a test fails; the caller
 // then runs the eigensolver.
 constexpr int kCholMaxR = 64;

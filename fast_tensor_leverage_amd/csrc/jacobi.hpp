@@ -294,8 +294,10 @@ __device__ __forceinline__ int jacobi_open(const double* A, int LD, int R) {
 // number, so that an item costs its entries and one {c, s} pair per rotation in
 // LDS traffic, which bounds a round from R = 48 on.  The operations on every
 // entry and their order are those of the two-barrier form: a pair whose top is
-// its larger index only has the sign of its s turned.  R = 64, Gaussian /
-// ill-conditioned factors: see k_gram_pinv.  Vout may be A1; A0 is overwritten.
+// its larger index only has the sign of its s turned.  k_gram_pinv over 700- and
+// 300-row Gaussian / ill-conditioned factors, two barriers a round -> this (us):
+// R = 32 156 / 296 -> 113 / 203, R = 16 59 / 123 -> 45 / 91.  Vout may be A1; A0 is
+// overwritten.
 template <int BS>
 __device__ __forceinline__ bool jacobi_small(double* A0, double* A1, double* V, int R, double* lam, double* Vout,
                                              JacobiShared& js, double* diag_tmp) {

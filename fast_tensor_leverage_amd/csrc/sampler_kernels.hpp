@@ -1187,9 +1187,9 @@ struct DrawCfg {
     static constexpr int EPL = VEC * NLD;                            // packed entries per lane
     static constexpr int HPL = (RMAX + SG - 1) / SG;   // vector entries per lane
     static constexpr int RPL = (RMAX + SG - 1) / SG;   // leaf rows per lane (scan)
-    // leaf dot products: LPR lanes per row, 8 columns per lane
+    // leaf dot products: LPR lanes per row (a power of two), 8 columns per lane
     static constexpr int LCOLS = 8;
-    static constexpr int LPR = RMAX / LCOLS;
+    static constexpr int LPR = RMAX <= 8 ? 1 : RMAX <= 16 ? 2 : RMAX <= 32 ? 4 : RMAX <= 64 ? 8 : 16;
     static constexpr int RPP = SG / LPR;                // rows per pass
 };
 
@@ -1334,13 +1334,67 @@ __device__ inline void descend_from(const ModeDev& md, const Shape& sh, uint32_t
     }
 }
 
+// The columns of lane `sub` of the LPR lanes of a leaf row, as 16-byte vectors:
+// vector q holds columns W (sub + LPR q) .. + W - 1, so the lanes of a row read
+// 16 LPR consecutive bytes per load (rows of odd length are aligned to their
+// elements only).  A vector that would pass the row's end ends there instead,
+// and leaf_coefs gives zero for its columns before W (sub + LPR q).  Eight
+// consecutive columns per lane touched as many 64-byte segments as there are
+// lanes, with each load: half the L1 accesses of a draw at R = 25.
+// R <= 16 (rows of two or one segments) keeps eight consecutive columns, whole
+// vectors at R = RMAX, else elements with the column clamped, x being zero past
+// R: vectors cost a draw 1.2% there (571 / 578 us, six modes, R = 16).
+template <typename TU, int RMAX, int LC, int LPR>
+__device__ inline void leaf_row(const TU* row, int R, int sub, TU (&buf)[LC]) {
+    constexpr int W = 16 / sizeof(TU);
+    typedef TU V __attribute__((ext_vector_type(W), aligned(sizeof(TU))));
+    constexpr bool CONSECUTIVE = RMAX <= 16;
+    if (R == LC * LPR) {
+#pragma unroll
+        for (int q = 0; q < LC / W; q++) {
+            const V v = *reinterpret_cast<const V*>(row + (CONSECUTIVE ? LC * sub + W * q : W * (sub + LPR * q)));
+#pragma unroll
+            for (int w = 0; w < W; w++) buf[q * W + w] = v[w];
+        }
+        return;
+    }
+    // formed per pass: hoisted, the offsets would hold registers through every
+    // descent of the kernel
+    asm volatile("" : "+v"(sub));
+    if constexpr (CONSECUTIVE) {
+#pragma unroll
+        for (int w = 0; w < LC; w++) buf[w] = row[min(LC * sub + w, R - 1)];
+    } else {
+#pragma unroll
+        for (int q = 0; q < LC / W; q++) {
+            const V v = *reinterpret_cast<const V*>(row + min(W * (sub + LPR * q), R - W));
+#pragma unroll
+            for (int w = 0; w < W; w++) buf[q * W + w] = v[w];
+        }
+    }
+}
+
+template <int RMAX, int W, int LC, int LPR>
+__device__ inline void leaf_coefs(const double* xs, int R, int sub, double (&xc)[LC]) {
+    if (RMAX <= 16 || R == LC * LPR) {
+#pragma unroll
+        for (int q = 0; q < LC; q++) xc[q] = xs[RMAX <= 16 ? LC * sub + q : W * (sub + LPR * (q / W)) + q % W];
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < LC / W; q++) {
+        const int b = W * (sub + LPR * q), at = min(b, R - W);
+#pragma unroll
+        for (int w = 0; w < W; w++) xc[q * W + w] = at + w >= b ? xs[at + w] : 0.0;
+    }
+}
+
 // Leaf row scan (partition_tree.hpp:336-391): q_t = (U_t . x)^2 for the rows
 // of the leaf, inclusive prefix over the group, P_{t+1} = prefix_t / total,
 // result = first t <= F-2 with frac < P_{t+1}, else F-1 (clamped to the last
 // real row of a partial leaf).
-// The dot products take LPR lanes per row, 8 consecutive columns per lane
-// (16-byte loads when R == RMAX, else element loads with the column clamped,
-// x being zero past R), summed over the LPR lanes with the DPP butterfly, and
+// The dot products take LPR lanes per row, 8 columns per lane (leaf_row),
+// summed over the LPR lanes with the DPP butterfly, and
 // RPP = SG / LPR rows per pass; q goes to LDS (qs, RMAX entries per group)
 // and lane g then owns rows g, g+SG, ... for the scan.  Few registers per
 // lane: the kernel's occupancy, not its bandwidth, bounds the descents.
@@ -1349,10 +1403,7 @@ __device__ inline uint32_t leaf_scan(const TU* __restrict__ U, uint64_t r0, uint
                                      int R, const double* xs, double* qs, double frac, int g, int lane) {
     using Cfg = DrawCfg<RMAX, SG>;
     constexpr int LC = Cfg::LCOLS, LPR = Cfg::LPR, RPP = Cfg::RPP, RPL = Cfg::RPL;
-    constexpr int W = 16 / sizeof(TU);
-    typedef TU V __attribute__((ext_vector_type(W)));
     const int sub = g % LPR, rsub = g / LPR;
-    const int col0 = sub * LC;
     const uint32_t passes = (F + RPP - 1) / RPP;
     // the loads of up to PCH passes are in flight together
     constexpr int PMAX = (RMAX + RPP - 1) / RPP;
@@ -1364,33 +1415,17 @@ __device__ inline uint32_t leaf_scan(const TU* __restrict__ U, uint64_t r0, uint
             const uint32_t t = (p0 + pp) * RPP + rsub;
             const uint32_t tc = t < rows ? t : rows - 1;
             const TU* row = U + (r0 + tc) * (uint64_t)R;
-            if (R == RMAX) {
-                const V* rv = reinterpret_cast<const V*>(row + col0);
-#pragma unroll
-                for (int q = 0; q < LC / W; q++) {
-                    const V v = rv[q];
-#pragma unroll
-                    for (int w = 0; w < W; w++) buf[pp][q * W + w] = v[w];
-                }
-            } else {
-                // formed per pass: hoisted, the eight clamped offsets would
-                // hold registers through every descent of the kernel
-                int cb = col0;
-                asm volatile("" : "+v"(cb));
-#pragma unroll
-                for (int w = 0; w < LC; w++) {
-                    const int b = cb + w;
-                    buf[pp][w] = row[b < R ? b : R - 1];
-                }
-            }
+            leaf_row<TU, RMAX, LC, LPR>(row, R, sub, buf[pp]);
         }
+        double xc[LC];  // read while the rows are on their way
+        leaf_coefs<RMAX, 16 / sizeof(TU), LC, LPR>(xs, R, sub, xc);
 #pragma unroll
         for (int pp = 0; pp < PCH; pp++) {
             double acc0 = 0.0, acc1 = 0.0;
 #pragma unroll
             for (int w = 0; w < LC; w += 2) {
-                acc0 += (double)buf[pp][w] * xs[col0 + w];
-                acc1 += (double)buf[pp][w + 1] * xs[col0 + w + 1];
+                acc0 += (double)buf[pp][w] * xc[w];
+                acc1 += (double)buf[pp][w + 1] * xc[w + 1];
             }
             const double d = group_sum<LPR>(acc0 + acc1);
             const uint32_t t = (p0 + pp) * RPP + rsub;
@@ -1541,7 +1576,12 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
         const int ra = g + SG * q;
         if (ra < R) {
             double y = 0.0;
-            for (int b = 0; b < R; b++) y += a.pinv[ra * R + b] * xs[b];
+            if constexpr (RMAX <= 16) {
+                for (int b = 0; b < R; b++) y += a.pinv[ra * R + b] * xs[b];
+            } else {  // symmetric: the lanes read a row (a column's entries lie in R lines)
+#pragma unroll 4
+                for (int b = 0; b < R; b++) y += a.pinv[b * R + ra] * xs[b];
+            }
             part += h[q] * y;
         }
     }
@@ -1557,8 +1597,12 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
     wave_sync_lds();
 }
 
+// Four waves per SIMD at R <= 32: three samples' chains in flight took 214 us
+// where four take 192 (I = 2^21, R = 32, J = 8192).  Not after the tile kernels,
+// whose rest of a descent waits for HBM and lost 7% to the narrower allocation
+// (I = 2^23, FP32: 835 / 775 us a call).
 template <int RMAX, int SG, int BS, bool USE32, bool RESUME>
-__global__ void __launch_bounds__(BS) k_krp_draw(DrawArgs a) {
+__global__ void __launch_bounds__(BS, !RESUME && SG == 32 && RMAX <= 32 ? 4 : 1) k_krp_draw(DrawArgs a) {
     using Cfg = DrawCfg<RMAX, SG>;
     constexpr int GPW = 64 / SG;  // groups per wave
     __shared__ double lds_x[BS / SG][RMAX];
@@ -1588,7 +1632,7 @@ __global__ void __launch_bounds__(BS) k_krp_draw(DrawArgs a) {
 // draws them with its request's arguments (fused: every sampled mode, then
 // the weight).  Each request's samples are those of its own k_krp_draw.
 template <int RMAX, int SG, int BS, bool USE32>
-__global__ void __launch_bounds__(BS) k_krp_draw_packed(const DrawArgs* __restrict__ reqs,
+__global__ void __launch_bounds__(BS, SG == 32 && RMAX <= 32 ? 4 : 1) k_krp_draw_packed(const DrawArgs* __restrict__ reqs,
                                                         const uint64_t* __restrict__ item_off, uint32_t n_req,
                                                         int R) {
     using Cfg = DrawCfg<RMAX, SG>;
@@ -1768,7 +1812,8 @@ __global__ void __launch_bounds__(BS) k_krp_draw_wave(DrawArgs a) {
             const int ra = lane + 64 * q;
             if (ra < R) {
                 double y = 0.0;
-                for (int b = 0; b < R; b++) y += a.pinv[ra * R + b] * xs[b];
+#pragma unroll 8
+                for (int b = 0; b < R; b++) y += a.pinv[b * R + ra] * xs[b];  // symmetric: the lanes read a row
                 part += h[q] * y;
             }
         }
@@ -1873,11 +1918,8 @@ __device__ inline uint32_t leaf_scan_block(const TU* __restrict__ U, uint64_t r0
     constexpr int LC = 8, LPR = RMAX / LC, RPP = BS / LPR;
     constexpr int PMAX = (RMAX + RPP - 1) / RPP;
     constexpr int PCH = PMAX < 4 ? PMAX : 4;
-    constexpr int W = 16 / sizeof(TU);
-    typedef TU V __attribute__((ext_vector_type(W)));
     const int tid = threadIdx.x;
     const int sub = tid % LPR, rsub = tid / LPR;
-    const int col0 = sub * LC;
     const uint32_t passes = (F + RPP - 1) / RPP;
     for (uint32_t p0 = 0; p0 < passes; p0 += PCH) {
         TU buf[PCH][LC];
@@ -1886,29 +1928,17 @@ __device__ inline uint32_t leaf_scan_block(const TU* __restrict__ U, uint64_t r0
             const uint32_t t = (p0 + pp) * RPP + rsub;
             const uint32_t tc = t < rows ? t : rows - 1;
             const TU* row = U + (r0 + tc) * (uint64_t)R;
-            if (R == RMAX) {
-                const V* rv = reinterpret_cast<const V*>(row + col0);
-#pragma unroll
-                for (int q = 0; q < LC / W; q++) {
-                    const V v = rv[q];
-#pragma unroll
-                    for (int w = 0; w < W; w++) buf[pp][q * W + w] = v[w];
-                }
-            } else {
-#pragma unroll
-                for (int w = 0; w < LC; w++) {
-                    const int b = col0 + w;
-                    buf[pp][w] = row[b < R ? b : R - 1];
-                }
-            }
+            leaf_row<TU, RMAX, LC, LPR>(row, R, sub, buf[pp]);
         }
+        double xc[LC];  // read while the rows are on their way
+        leaf_coefs<RMAX, 16 / sizeof(TU), LC, LPR>(xs, R, sub, xc);
 #pragma unroll
         for (int pp = 0; pp < PCH; pp++) {
             double acc0 = 0.0, acc1 = 0.0;
 #pragma unroll
             for (int w = 0; w < LC; w += 2) {
-                acc0 += (double)buf[pp][w] * xs[col0 + w];
-                acc1 += (double)buf[pp][w + 1] * xs[col0 + w + 1];
+                acc0 += (double)buf[pp][w] * xc[w];
+                acc1 += (double)buf[pp][w + 1] * xc[w + 1];
             }
             const double d = group_sum<LPR>(acc0 + acc1);
             const uint32_t t = (p0 + pp) * RPP + rsub;

@@ -186,8 +186,13 @@ void* ftl_sampler_stream(ftl_sampler* s);
  * sample per block above; 1 = one sample per wave, R <= 32; 2 = one sample
  * per block, R > 32; 3 = a group of lanes per sample at any rank),
  * "block_threads" (threads per block of the one-sample-per-block kernel:
- * 128/256/512, 0 = 256), "xcd_buckets" (1: descents bucketed by level-3
- * subtree onto XCD-affine blocks, R <= 64), "overlap_compute_m" (1, the
+ * 128/256/512, 0 = 256), "sample_order" (order in which the draw kernels take
+ * the samples: 0 = by index, 1 = by Gram uniform, a contiguous part per XCD,
+ * 2 = 1 where it pays, the default; J <= 2^24), "xcd_buckets" (1 sets
+ * "sample_order" 1, 0 sets 2), "tile_descent" (eigen descents and upper Gram
+ * levels of 16 ordered samples per wave on the FP64 matrix cores: 0 never,
+ * 1 with "mode_split" and J <= 2^24, 2 = 1 where it pays, the default),
+ * "overlap_compute_m" (1, the
  * default for a sampler with a stream of its own: computeM of a call runs on
  * a second stream into one of two buffer sets, overlapping the previous
  * call's draw kernels; 0: computeM and draw in order on one stream).
