@@ -1179,12 +1179,12 @@ struct Sampler {
     // Calls f(RMAX, SG) (as integral constants) for the draw configuration of
     // this sampler.  Measured at N=3, I=2^23, R=32, J=5e4: SG=32 fastest for
     // both precisions (FP64 1.56 ms vs 1.64 at SG=16; FP32 1.15 vs 1.33).
-    // RMAX 21, 27 and 48: a node is read with four or six loads a lane instead
-    // of nine, ten instead of 17, and held in as many fewer registers.  Draws
-    // with the wider class and now (us): three modes of 2^20, J = 50,000, R = 20
-    // 641 / 500; 2^18, J = 20,000, R = 48 992 / 574, R = 40 930 / 558; with the
-    // leaf rows' loads of leaf_row, 183 x 24 x 1140 x 1717, J = 65,536, R = 25
-    // 567 / 405.
+    // RMAX 21, 27, 40, 48 and 56: a node is read with four or six loads a lane
+    // instead of nine, seven, ten or 13 instead of 17, and held in as many fewer
+    // registers.  Draws with the wider class and now (us): three modes of 2^20, J
+    // = 50,000, R = 20 641 / 500; 2^18, J = 20,000, R = 36 557 / 479, R = 48 992 /
+    // 574, R = 52 932 / 694; with the leaf rows' loads of leaf_row, 183 x 24 x 1140
+    // x 1717, J = 65,536, R = 25 567 / 405.
     template <typename F>
     void with_cfg(F&& f) const {
         using std::integral_constant;
@@ -1203,7 +1203,9 @@ struct Sampler {
             else f(integral_constant<int, 32>{}, integral_constant<int, 32>{});
         } else if (R <= 64) {
             if (sg == 32) f(integral_constant<int, 64>{}, integral_constant<int, 32>{});
+            else if (R <= 40) f(integral_constant<int, 40>{}, integral_constant<int, 64>{});
             else if (R <= 48) f(integral_constant<int, 48>{}, integral_constant<int, 64>{});
+            else if (R <= 56) f(integral_constant<int, 56>{}, integral_constant<int, 64>{});
             else f(integral_constant<int, 64>{}, integral_constant<int, 64>{});
         } else {
             f(integral_constant<int, 128>{}, integral_constant<int, 64>{});

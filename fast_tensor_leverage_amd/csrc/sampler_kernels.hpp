@@ -1597,12 +1597,19 @@ __device__ __forceinline__ void krp_draw_item(const DrawArgs& a, uint64_t item, 
     wave_sync_lds();
 }
 
-// Four waves per SIMD at R <= 32: three samples' chains in flight took 214 us
-// where four take 192 (I = 2^21, R = 32, J = 8192).  Not after the tile kernels,
-// whose rest of a descent waits for HBM and lost 7% to the narrower allocation
-// (I = 2^23, FP32: 835 / 775 us a call).
+// Waves per SIMD of the group kernels.  Four at R <= 32: three samples' chains in
+// flight took 214 us where four take 192 (I = 2^21, R = 32, J = 8192).  Three at R
+// = 49-56 FP32, a few registers under what the compiler takes: 798 / 714 us at R =
+// 52, J = 20,000 (FP64 takes 165 and has them: 694, bounded 733).
+// Not where it spills (R = 64 at three 940 / 1,039, R = 48 at four 574 / 638), and
+// not after the tile kernels, whose rest of a descent waits for HBM (I = 2^23, R =
+// 32 FP32 775 / 835 us a call).
+constexpr int draw_waves(int rmax, int sg, bool fp32) {
+    return sg == 32 && rmax <= 32 ? 4 : sg == 64 && rmax == 56 && fp32 ? 3 : 1;
+}
+
 template <int RMAX, int SG, int BS, bool USE32, bool RESUME>
-__global__ void __launch_bounds__(BS, !RESUME && SG == 32 && RMAX <= 32 ? 4 : 1) k_krp_draw(DrawArgs a) {
+__global__ void __launch_bounds__(BS, RESUME ? 1 : draw_waves(RMAX, SG, USE32)) k_krp_draw(DrawArgs a) {
     using Cfg = DrawCfg<RMAX, SG>;
     constexpr int GPW = 64 / SG;  // groups per wave
     __shared__ double lds_x[BS / SG][RMAX];
@@ -1632,7 +1639,7 @@ __global__ void __launch_bounds__(BS, !RESUME && SG == 32 && RMAX <= 32 ? 4 : 1)
 // draws them with its request's arguments (fused: every sampled mode, then
 // the weight).  Each request's samples are those of its own k_krp_draw.
 template <int RMAX, int SG, int BS, bool USE32>
-__global__ void __launch_bounds__(BS, SG == 32 && RMAX <= 32 ? 4 : 1) k_krp_draw_packed(const DrawArgs* __restrict__ reqs,
+__global__ void __launch_bounds__(BS, draw_waves(RMAX, SG, USE32)) k_krp_draw_packed(const DrawArgs* __restrict__ reqs,
                                                         const uint64_t* __restrict__ item_off, uint32_t n_req,
                                                         int R) {
     using Cfg = DrawCfg<RMAX, SG>;

@@ -1,6 +1,6 @@
 """Draws at the edges of the rank classes and of the leaf rows' vector loads:
-R on either side of 8, 16, 21, 27, 32, 48 and 64, odd and even, with FP64 and
-FP32 leaves, from factors whose leaves are full, partial and of one row.
+R on either side of 8, 16, 21, 27, 32, 40, 48, 56 and 64, odd and even, with FP64
+and FP32 leaves, from factors whose leaves are full, partial and of one row.
 Indices equal those of the one-sample-per-wave kernel (R <= 32) or of the
 block kernel, and of the CPU sampler in FP64."""
 import numpy as np
@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
-@pytest.mark.parametrize("R", [1, 2, 3, 4, 8, 9, 15, 16, 17, 20, 21, 22, 26, 27, 28, 31, 32, 33, 47, 48, 49, 63, 64, 65,
-                               67, 127])
+@pytest.mark.parametrize("R", [1, 2, 3, 4, 8, 9, 15, 16, 17, 20, 21, 22, 26, 27, 28, 31, 32, 33, 40, 41, 47, 48, 49, 56,
+                               57, 63, 64, 65, 67, 127])
 def test_rank_classes(oracle, R, precision):
     import fast_tensor_leverage_amd as ftl
     print(f"[gpu] rank classes R={R} {precision}", flush=True)
