@@ -1282,11 +1282,18 @@ struct Sampler {
     // FP32 1.46 / 2.09 ms; R = 128, J = 8192 2.35 / 2.32 ms.  Up to R = 64 the
     // group kernel reads a third as much per sample and a tile's chain of
     // dependent matrix products is the longer one unless each SIMD has two
-    // tiles or more: J = 50,000, R = 33 1.56 / 2.23 ms, R = 64 2.11 / 2.47 ms, R
-    // = 32 (I = 2^22, two modes) 566 / 602 us, but J = 20,011, R = 64 1.14 / 1.09
-    // ms and J = 8192, R = 48 515 / 485 us.  R <= 16 leaves most of a 16 x 16
-    // block empty: 531 / 455 us.
-    bool tiles_pay() const { return R > 64 ? J >= 8192 : R > 16 && J >= 32768; }
+    // tiles or more, and the rank is not far below the tiles' multiple of 16 where
+    // the group kernel's class fits it (22-27, 49-56).  I = 2^19 FP64, us, tiles /
+    // groups: J = 32768 R = 32 438 / 514, R = 36 775 / 785 (FP32 749 / 818), R = 44
+    // 850 / 952, R = 64 1,340 / 1,588; J = 20,011, R = 64 1.14 / 1.09 ms.  R = 25
+    // and R = 52 at J = 50,000 557 / 541 and 1,806 / 1,693, at J = 65536 653 / 677
+    // and 2,127 / 2,142.  Never at R <= 21 (R = 20, J = 65536 535 / 504) nor R <=
+    // 16, which leaves most of a block empty: 531 / 455 us.
+    bool tiles_pay() const {
+        if (R > 64) return J >= 8192;
+        if (R <= 27 || (R > 48 && R <= 56)) return R > 21 && J >= 65536;
+        return J >= 32768;
+    }
     bool tiled(const std::vector<int>& order) const {
         if (!st_s || !mode_split || tile_descent == 0) return false;
         for (int k : order)
