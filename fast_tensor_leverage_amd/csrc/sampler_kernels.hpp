@@ -1060,13 +1060,16 @@ struct DrawArgs {
 // neighbouring subtrees one after the other: waves that run at the same time
 // then read the same nodes, and the order is cut into one contiguous part per
 // XCD (ordered_block), so that each L2 sees an eighth of the tree and fetches a
-// node once instead of once per XCD and eviction.  A sample's result does not
-// depend on its place, so only a counting sort by the uniform's leading bits
-// is needed (the order inside a bin is arbitrary), for every sampled mode of
-// the call at once, beside computeM.  Blocks of the sort count their share of
-// the samples in LDS and write the counts out; the second kernel's blocks each
-// sum the table up to their own entries (device-scope atomics on one table
-// took 34 us for three modes of 50,000 samples, most of it their round trips).
+// node once instead of once per XCD and eviction.  A counting sort by the
+// uniform's leading bits is enough, for every sampled mode of the call at once,
+// beside computeM.  It is stable: samples of a bin follow one another by index,
+// so the order is a function of the uniforms alone.  The draw kernels need that
+// after the tile kernels: the level at which a sample leaves its tile depends on
+// the other samples of the tile, and the kernels on either side round a node's
+// mass differently.  Blocks of the sort count their share of the samples in LDS
+// and write the counts out; the second kernel's blocks each sum the table up to
+// their own entries (device-scope atomics on one table took 34 us for three
+// modes of 50,000 samples, most of it their round trips).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kOrderBins = 4096;
 constexpr uint32_t kOrderMaxBlocks = 256;
@@ -1114,11 +1117,39 @@ __global__ void __launch_bounds__(256) k_order_count(OrderArgs a) {
     for (uint32_t b = threadIdx.x; b < kOrderBins; b += 256) out[b] = cnt[b];
 }
 
+// A wave places a contiguous quarter of the block's share, 64 samples at a time
+// in index order: a sample's place is its bin's next one for the wave plus the
+// number of lower lanes with the same bin.  One entry more per 16 bins, the bins
+// of a thread in the scan, keeps its threads on different LDS banks.
+__device__ inline uint32_t order_slot(uint32_t bin) { return bin + bin / 16; }
+
 __global__ void __launch_bounds__(256) k_order_scatter(OrderArgs a) {
     constexpr int PT = kOrderBins / 256;
-    __shared__ uint32_t at[kOrderBins];
+    constexpr int AH = 8;  // bins loaded ahead
+    constexpr uint32_t SLOTS = kOrderBins + kOrderBins / 16;
+    static_assert(PT == 16, "order_slot");
+    __shared__ alignas(16) uint32_t at[4][SLOTS];
     __shared__ uint32_t wsum[4];
     const uint32_t t = blockIdx.y;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint16_t* bin = a.bin + t * a.J;
+    const uint64_t i0 = min((uint64_t)blockIdx.x * a.share + (uint64_t)w * (a.share / 4), a.J);
+    const uint64_t i1 = min(i0 + a.share / 4, a.J);
+    // the bins of 64 AH samples at a time; the first ones (all of them up to J =
+    // 2^19) stay in registers between the count and the placing
+    uint32_t b[AH];
+    auto fetch = [&](uint64_t from) {
+#pragma unroll
+        for (int u = 0; u < AH; u++) b[u] = bin[min(from + 64 * u + lane, a.J - 1)];
+    };
+    fetch(i0);
+    for (uint32_t e = threadIdx.x; e < SLOTS; e += 256) reinterpret_cast<uint4*>(at)[e] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < AH; u++)
+        if (i0 + 64 * u + lane < i1) atomicAdd(&at[w][order_slot(b[u])], 1u);
+#pragma unroll 8
+    for (uint64_t i = i0 + 64 * AH + lane; i < i1; i += 64) atomicAdd(&at[w][order_slot(bin[i])], 1u);
     // bins PT * threadIdx.x + q: their samples in all blocks, and in the
     // blocks before this one
     uint32_t all[PT], before[PT];
@@ -1145,7 +1176,6 @@ __global__ void __launch_bounds__(256) k_order_scatter(OrderArgs a) {
         before[q] += run;
         run += all[q];
     }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     uint32_t incl = run;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -1157,13 +1187,38 @@ __global__ void __launch_bounds__(256) k_order_scatter(OrderArgs a) {
     uint32_t base = incl - run;
     for (int q = 0; q < w; q++) base += wsum[q];
 #pragma unroll
-    for (int q = 0; q < PT; q++) at[threadIdx.x * PT + q] = base + before[q];
+    for (int q = 0; q < PT; q++) {
+        uint32_t pos = base + before[q];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            uint32_t* next = &at[v][order_slot(threadIdx.x * PT + q)];
+            const uint32_t n = *next;
+            *next = pos;
+            pos += n;
+        }
+    }
     __syncthreads();
-    const uint64_t i0 = (uint64_t)blockIdx.x * a.share, i1 = min(i0 + a.share, a.J);
-#pragma unroll 8
-    for (uint64_t i = i0 + threadIdx.x; i < i1; i += 256) {
-        const uint32_t pos = atomicAdd(at + a.bin[t * a.J + i], 1u);
-        a.perm[t * a.J + pos] = (uint32_t)i;
+    const uint64_t below = (1ull << lane) - 1;
+    for (uint64_t base_i = i0; base_i < i1; base_i += 64 * AH) {
+        if (base_i > i0) fetch(base_i);
+#pragma unroll
+        for (int u = 0; u < AH; u++) {
+            const uint64_t i = base_i + 64 * u + lane;
+            const bool in = i < i1;
+            uint64_t same = __ballot(in);
+#pragma unroll
+            for (uint32_t bit = 1; bit < kOrderBins; bit <<= 1) {
+                const uint64_t set = __ballot((b[u] & bit) != 0);
+                same &= b[u] & bit ? set : ~set;
+            }
+            const uint32_t rank = __popcll(same & below), n = __popcll(same);
+            uint32_t* next = &at[w][order_slot(b[u])];
+            const uint32_t pos = *next;
+            wave_sync_lds();
+            if (in && rank + 1 == n) *next = pos + n;
+            wave_sync_lds();
+            if (in) a.perm[t * a.J + pos + rank] = (uint32_t)i;
+        }
     }
 }
 
