@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(HERE, LIB_NAME)
 
 SOURCES = ["sampler.hip", "als.hip", "serve.hip"]
 HEADERS = ["ftl_common.hpp", "sampler_kernels.hpp", "tile_kernels.hpp", "als_kernels.hpp", "jacobi.hpp", "wave_ops.hpp",
-           "sampler_internal.hpp"]
+           "sampler_internal.hpp", "factor_source.hpp"]
 
 ARCH = os.environ.get("FTL_OFFLOAD_ARCH", "gfx950")
 

@@ -16,6 +16,7 @@
 #include <mutex>
 #include <sstream>
 
+#include "factor_source.hpp"
 #include "ftl_common.hpp"
 #include "sampler_internal.hpp"
 #include "sampler_kernels.hpp"
@@ -618,6 +619,27 @@ struct Sampler {
         }
     }
 
+    // Where build_mode reads a new factor of mode m: device memory that a kernel
+    // of this GPU can read as it is, else null after queueing its copy to U64.
+    const double* stage_factor(const ModeHost& m, const double* U, bool on_device) {
+        const uint64_t bytes = m.I * R * sizeof(double);
+        if (on_device) {
+            hipPointerAttribute_t at{};
+            hipDeviceptr_t base = nullptr;
+            size_t size = 0;
+            if (hipPointerGetAttributes(&at, U) == hipSuccess && at.type == hipMemoryTypeDevice &&
+                hipMemGetAddressRange(&base, &size, const_cast<double*>(U)) == hipSuccess) {
+                const FactorMemory fm{true, at.device, (uint64_t)(uintptr_t)base, size};
+                if (factor_in_place(fm, device, (uint64_t)(uintptr_t)U, bytes)) return U;
+            } else {
+                (void)hipGetLastError();  // memory unknown to the runtime: the copy decides
+            }
+        }
+        FTL_HIP_CHECK(hipMemcpyAsync(m.U64, U, bytes, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
+                                     stream));
+        return nullptr;
+    }
+
     // Builds on a stream other than the sampler's own occur only for samplers
     // on a borrowed stream, which keep one computeM set on that stream.
     // src: the factor to build from (device), copied to U64 on the way; null: U64.
@@ -957,13 +979,11 @@ struct Sampler {
                 m.U64 = const_cast<double*>(U[k]);
             } else {
                 m.U64 = dalloc<double>(m.I * R);
-                if (!on_device)
-                    FTL_HIP_CHECK(hipMemcpyAsync(m.U64, U[k], m.I * R * sizeof(double), hipMemcpyHostToDevice,
-                                                 stream));
             }
+            const double* src = alias ? nullptr : stage_factor(m, U[k], on_device);
             alloc_trees(m);
             if (precision == FTL_FP32) m.U32 = dalloc<float>(m.I * R);
-            build_mode(k, nullptr, on_device && !alias ? U[k] : nullptr);
+            build_mode(k, nullptr, src);
         }
         const uint64_t R2 = R * R;
         etree_nodes = (uint32_t)(2 * R - 1);
@@ -1050,9 +1070,7 @@ struct Sampler {
         FTL_REQUIRE(Uj != nullptr, "update_sampler: null factor");
         ModeHost& m = modes[j];
         wait_foreign_draws();
-        if (!on_device)
-            FTL_HIP_CHECK(hipMemcpyAsync(m.U64, Uj, m.I * R * sizeof(double), hipMemcpyHostToDevice, stream));
-        build_mode(j, nullptr, on_device ? Uj : nullptr);
+        build_mode(j, nullptr, stage_factor(m, Uj, on_device));
     }
 
     std::vector<int> sampled_modes(uint32_t j) const {
