@@ -108,8 +108,8 @@ __host__ __device__ inline uint32_t node_depth(uint64_t c) {
 // Packed upper triangle: element (a, b), a <= b, of an R x R symmetric matrix
 // sits at a*R - a*(a-1)/2 + (b - a).  Node strides are rounded up so every
 // node starts on a 128-byte line.
-__host__ __device__ inline uint64_t tri_size(uint64_t R) { return R * (R + 1) / 2; }
-__host__ __device__ inline uint64_t tri_stride64(uint64_t R) { return (tri_size(R) + 15) / 16 * 16; }
+__host__ __device__ constexpr uint64_t tri_size(uint64_t R) { return R * (R + 1) / 2; }
+__host__ __device__ constexpr uint64_t tri_stride64(uint64_t R) { return (tri_size(R) + 15) / 16 * 16; }
 __host__ __device__ inline uint64_t tri_stride32(uint64_t R) { return (tri_size(R) + 31) / 32 * 32; }
 __host__ __device__ inline uint64_t tri_offset(uint64_t R, uint64_t a, uint64_t b) {
     return a * R - a * (a - 1) / 2 + (b - a);

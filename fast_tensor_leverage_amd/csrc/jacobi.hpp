@@ -56,12 +56,19 @@ __device__ inline void jacobi_pair(int k, int round, int n2, int& p, int& q) {
     }
 }
 
-// Rotation (c, s) annihilating apq = A[p][q]; false (c = 1, s = 0) when it is
-// negligible.
-__device__ inline bool jacobi_rotation(double app, double aqq, double apq, double& c, double& s) {
+// The rotation of tangent t != 0.
+__device__ inline void jacobi_cs(double t, double& c, double& s) {
+#pragma clang fp contract(off)
+    c = fast_rsq(1.0 + t * t);
+    s = t * c;
+}
+
+// Rotation (c, s) of tangent t annihilating apq = A[p][q]; false (c = 1, s = t = 0)
+// when it is negligible.
+__device__ inline bool jacobi_rotation(double app, double aqq, double apq, double& c, double& s, double& t) {
 #pragma clang fp contract(off)
     c = 1.0;
-    s = 0.0;
+    s = t = 0.0;
     const double eps = 2.220446049250313e-16;
     // |apq| <= eps sqrt(|app aqq|), compared in squares (no square root on
     // the round's critical path)
@@ -70,7 +77,6 @@ __device__ inline bool jacobi_rotation(double app, double aqq, double apq, doubl
     // Newton step (error ~1 ulp; the rotation stays orthogonal to working
     // precision)
     const double tau = (aqq - app) * fast_rcp(2.0 * apq);
-    double t;
     if (fabs(tau) > 1e150) {
         t = 0.5 * fast_rcp(tau);
     } else {
@@ -78,8 +84,7 @@ __device__ inline bool jacobi_rotation(double app, double aqq, double apq, doubl
         const double sq = x * fast_rsq(x);
         t = (tau >= 0 ? 1.0 : -1.0) * fast_rcp(fabs(tau) + sq);
     }
-    c = fast_rsq(1.0 + t * t);
-    s = t * c;
+    jacobi_cs(t, c, s);
     return true;
 }
 
@@ -88,7 +93,8 @@ __device__ inline bool jacobi_rotation(const double* A, int LD, int R, int p, in
     c = 1.0;
     s = 0.0;
     if (q >= R) return false;
-    return jacobi_rotation(A[p * LD + p], A[q * LD + q], A[p * LD + q], c, s);
+    double t;
+    return jacobi_rotation(A[p * LD + p], A[q * LD + q], A[p * LD + q], c, s, t);
 }
 
 // Returns false (in every thread) when the sweep cap ended the iteration
@@ -132,7 +138,7 @@ __device__ __forceinline__ void jacobi_sorted(const double* A, int LD, const dou
 // The order the matrix is padded to (a zero row and column when odd) and the
 // row length of A: odd, so rows start in different LDS banks.  Above
 // kJacobiSmallR the general solver's A is not padded.
-__host__ __device__ inline int jacobi_n2(int R) { return R + (R & 1); }
+__host__ __device__ constexpr int jacobi_n2(int R) { return R + (R & 1); }
 __host__ __device__ inline int jacobi_ld(int R) { return R <= kJacobiSmallR ? jacobi_n2(R) + 1 : R + 1; }
 
 // Element of pair k's top / bottom in round `round`, m = n2 - 1 rounds a sweep:
@@ -171,14 +177,13 @@ __device__ inline double jacobi_entry_after(const double* A, int LD, const doubl
 }
 
 // Rotation of pair k, whose elements in its round are P (top) and Q, to rot[k]
-// (and to log[k]); whether it is applied.
-__device__ __forceinline__ bool jacobi_put(double2* rot, double2* log, uint32_t k, int R, int P, int Q, double app,
+// (and its tangent, of the same sign, to log[k]); whether it is applied.
+__device__ __forceinline__ bool jacobi_put(double2* rot, double* log, uint32_t k, int R, int P, int Q, double app,
                                            double aqq, double apq) {
-    double c = 1.0, s = 0.0;
-    const bool act = max(P, Q) < R && jacobi_rotation(app, aqq, apq, c, s);
-    const double2 g = make_double2(c, P < Q ? s : -s);
-    rot[k] = g;
-    if (log) log[k] = g;
+    double c = 1.0, s = 0.0, t = 0.0;
+    const bool act = max(P, Q) < R && jacobi_rotation(app, aqq, apq, c, s, t);
+    rot[k] = make_double2(c, P < Q ? s : -s);
+    if (log) log[k] = P < Q ? t : -t;
     return act;
 }
 
@@ -187,7 +192,7 @@ __device__ __forceinline__ bool jacobi_put(double2* rot, double2* log, uint32_t 
 // its bottom the bottom of pair k - 1 (the first pair's the top of pair 1).
 __device__ __forceinline__ bool jacobi_next_rotation(const double* A, int LD, int R, const double2* rot,
                                                      uint32_t round, uint32_t m, uint32_t np, uint32_t k, double2* out,
-                                                     double2* log) {
+                                                     double* log) {
     const uint32_t rn = round + 1 == m ? 0 : round + 1;
     const int P = jacobi_top(k, rn, m), Q = jacobi_bottom(k, rn, m);
     uint32_t kp, sp, kq, sq;
@@ -390,29 +395,30 @@ __host__ __device__ inline uint64_t jacobi_solve_lds_doubles(uint64_t R) {
     const uint64_t n2 = (uint64_t)jacobi_n2((int)R);
     return (R <= (uint64_t)kJacobiDoubleR ? 2 : 1) * n2 * (n2 + 1);
 }
-// Doubles of a matrix's log of rotations.
-__host__ __device__ inline uint64_t jacobi_log_doubles(uint64_t R) {
+// Doubles of a matrix's log of rotations: their tangents, from which (c, s)
+// follow bit for bit, for every sweep up to the cap.
+__host__ __device__ constexpr uint64_t jacobi_log_doubles(uint64_t R) {
     const uint64_t n2 = (uint64_t)jacobi_n2((int)R);
-    return kJacobiMaxSweeps * (n2 - 1) * (n2 / 2) * 2;
+    return kJacobiMaxSweeps * (n2 - 1) * (n2 / 2);
 }
 
 // A (n2 x (n2 + 1), padding zero) diagonalised: lam ascending, rank[v] the place
-// of diagonal entry v, *rounds the rounds done and their rotations in log (n2 / 2
+// of diagonal entry v, *rounds the rounds done and their tangents in log (n2 / 2
 // per round).  TWO: A1 is the second buffer; else two barriers a round, in place.
 template <int BS, bool TWO>
-__device__ __forceinline__ void jacobi_solve(double* A0, double* A1, int R, double2* log, double* lam, int* rank,
+__device__ __forceinline__ void jacobi_solve(double* A0, double* A1, int R, double* log, double* lam, int* rank,
                                              int* rounds, JacobiShared& js, double* diag_tmp) {
     const int tid = threadIdx.x, wave = tid >> 6;
     const int n2 = jacobi_n2(R), LD = n2 + 1;
     const uint32_t m = n2 - 1, np = n2 / 2;
     int cur = 0;
     bool carry = false;
-    auto first = [&](const double* A, int buf, uint32_t round, double2* to) {
+    auto first = [&](const double* A, int buf, uint32_t round, double* to) {
         const int P = jacobi_top(tid, round, m), Q = jacobi_bottom(tid, round, m);
         const int p = min(P, Q), q = max(P, Q);
         return jacobi_put(js.rot[buf], to, tid, R, P, Q, A[p * LD + p], A[q * LD + q], A[p * LD + q]);
     };
-    double2* lg = log;  // the log of the round
+    double* lg = log;  // the log of the round
     if constexpr (TWO) {
         if (tid < (int)np) carry = first(A0, 0, 0, lg);
         __syncthreads();
@@ -482,27 +488,32 @@ __device__ inline double wave_from_prev(double v) { return dpp_f64<0x138>(v); }
 // the round, and hands them on to the neighbouring lanes.  put(v, x): entry x of
 // eigenvector column v.  V starts as the identity.
 template <int LPR, class Put>
-__device__ __forceinline__ void jacobi_row(const double2* log, int rounds, int R, int i, int lane, Put put) {
+__device__ __forceinline__ void jacobi_row(const double* log, int rounds, int R, int i, int lane, Put put) {
 #pragma clang fp contract(off)
     const uint32_t m = jacobi_n2(R) - 1, np = jacobi_n2(R) / 2;
     const uint32_t k = lane & (LPR - 1), kc = k < np ? k : np - 1;
     double x = jacobi_top(k, 0, m) == i ? 1.0 : 0.0, y = jacobi_bottom(k, 0, m) == i ? 1.0 : 0.0;
     if (k >= np) x = y = 0.0;
-    constexpr int AH = 8;  // rotations loaded ahead
-    double2 g[AH];
-    const double2* src = log + kc;
+    constexpr int AH = 8;  // tangents loaded ahead
+    double g[AH];
+    const double* src = log + kc;
 #pragma unroll
     for (int u = 0; u < AH; u++) g[u] = src[(uint64_t)min(u, rounds - 1) * np];
     for (int r0 = 0; r0 < rounds; r0 += AH) {
+        // off the chain of the rounds: a launch at R = 128 122 us, inside it 168
+        double c[AH], s[AH];
 #pragma unroll
         for (int u = 0; u < AH; u++) {
-            const double2 c = g[u];
+            jacobi_cs(g[u], c[u], s[u]);
             g[u] = src[(uint64_t)min(r0 + AH + u, rounds - 1) * np];
+        }
+#pragma unroll
+        for (int u = 0; u < AH; u++) {
             if (r0 + u < rounds) {
                 double xn = x, yn = y;
-                if (c.y != 0.0) {
-                    xn = c.x * x - c.y * y;
-                    yn = c.y * x + c.x * y;
+                if (s[u] != 0.0) {
+                    xn = c[u] * x - s[u] * y;
+                    yn = s[u] * x + c[u] * y;
                 }
                 if (np > 1) {
                     const double up = wave_from_next(xn), down = wave_from_prev(yn);

@@ -365,6 +365,14 @@ constexpr uint64_t kOrderMaxJ = 1ull << 24;
 
 inline uint64_t order_blocks(uint64_t J) { return (J + order_share(J) - 1) / order_share(J); }
 
+// Every solve's log fits the eigen tree that k_cm_solve keeps it in.
+constexpr bool cm_logs_fit() {
+    for (uint64_t R = kJacobiSplitR; R <= 128; R++)
+        if (jacobi_log_doubles(R) > (2 * R - 1) * tri_stride64(R)) return false;
+    return true;
+}
+static_assert(cm_logs_fit(), "cm_log");
+
 struct Sampler {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -389,7 +397,6 @@ struct Sampler {
     // every computeM after the tree builds queued before it.
     struct MSet {
         double *pinv = nullptr, *W = nullptr, *E = nullptr, *etree = nullptr, *lam = nullptr;
-        double* log = nullptr;
         int* rank = nullptr;
         hipEvent_t cm_done = nullptr, draw_done = nullptr;
     };
@@ -993,10 +1000,7 @@ struct Sampler {
             ms.W = dalloc<double>(R2);
             ms.E = dalloc<double>(N * R2);
             ms.etree = dalloc<double>((uint64_t)N * etree_nodes * ts64 + pad);
-            if (R >= (uint64_t)kJacobiSplitR) {
-                ms.log = dalloc<double>((N + 1) * jacobi_log_doubles(R));
-                ms.rank = dalloc<int>((N + 1) * (R + 1));
-            }
+            if (R >= (uint64_t)kJacobiSplitR) ms.rank = dalloc<int>((N + 1) * (R + 1));
             ms.lam = dalloc<double>((uint64_t)(N + 1) * R);
             FTL_HIP_CHECK(hipMemsetAsync(ms.E, 0, N * R2 * sizeof(double), stream));
             FTL_HIP_CHECK(
@@ -1056,8 +1060,7 @@ struct Sampler {
         const uint64_t R2 = R * R;
         total += up(R2 * 8) * 2 + up(N * R2 * 8) + up(((uint64_t)N * (2 * R - 1) * ts64 + pad) * 8) +
                  up((uint64_t)(N + 1) * R * 8);
-        if (R >= (uint64_t)kJacobiSplitR)
-            total += up((N + 1) * jacobi_log_doubles(R) * 8) + up((N + 1) * (R + 1) * sizeof(int));
+        if (R >= (uint64_t)kJacobiSplitR) total += up((N + 1) * (R + 1) * sizeof(int));
         total += up(J * R * 8);
         if (J <= kOrderMaxJ)
             total += up(2 * N * J * 2) + up(2 * N * J * 4) + up(2 * N * order_blocks(J) * kOrderBins * 4) + up(J * 4) +
@@ -1090,7 +1093,6 @@ struct Sampler {
         a.W = ms.W;
         a.E = ms.E;
         a.etree = ms.etree;
-        a.log = reinterpret_cast<double2*>(ms.log);
         a.rank = ms.rank;
         a.lam_out = ms.lam;
         a.ts64 = ts64;

@@ -723,9 +723,8 @@ struct ComputeMArgs {
     double* E;       // N x R x R
     double* etree;   // N x etree_nodes x ts64
     double* lam_out; // (m+1) x R eigenvalues
-    // R >= kJacobiSplitR: per solve (the Gram's, then the sampled modes') its
-    // log of rotations, the places of its eigenvalues and its round count
-    double2* log;    // (m+1) x jacobi_log_doubles(R) / 2
+    // R >= kJacobiSplitR: per solve (the Gram's, then the sampled modes') the
+    // places of its eigenvalues and its round count
     int* rank;       // (m+1) x (R+1), the count last
     uint32_t ts64;
     uint32_t etree_nodes;
@@ -917,6 +916,15 @@ __device__ inline const ComputeMArgs& cm_sel(const ComputeMSel& s, bool gram, ui
     return s.many ? s.many[gram ? b : s.req[b]] : s.one;
 }
 
+// The log of rotations of solve t (-1: the Gram's): in the eigen tree of sampled
+// mode t (the first one's), which k_cm_etree writes whole after the last use.  A
+// tree of 2 R - 1 nodes holds it (checked in sampler.hip), so a sampler needs no
+// memory for logs; they stay off other modes' trees, whose first entries the draw
+// kernels read past a last node.
+__device__ inline double* cm_log(const ComputeMArgs& a, int t) {
+    return a.etree + (uint64_t)a.modes[t < 0 ? 0 : t] * a.etree_nodes * a.ts64;
+}
+
 template <int BS, bool TWO>
 __global__ void __launch_bounds__(BS) k_cm_solve(ComputeMSel sel, int gram) {
 #pragma clang fp contract(off)
@@ -932,8 +940,7 @@ __global__ void __launch_bounds__(BS) k_cm_solve(ComputeMSel sel, int gram) {
     __syncthreads();
     int* rank = a.rank + (uint64_t)(t + 1) * (R + 1);
     double* lam = a.lam_out + (uint64_t)(t + 1) * R;
-    double2* log = a.log + (uint64_t)(t + 1) * (jacobi_log_doubles(R) / 2);
-    jacobi_solve<BS, TWO>(smem, smem + n2 * LD, R, log, lam, rank, rank + R, js, diag_tmp);
+    jacobi_solve<BS, TWO>(smem, smem + n2 * LD, R, cm_log(a, t), lam, rank, rank + R, js, diag_tmp);
 }
 
 template <int LPR>
@@ -946,17 +953,15 @@ __global__ void __launch_bounds__(64) k_cm_vectors(ComputeMSel sel, int gram) {
     const int i = (int)(blockIdx.x * (64 / LPR) + threadIdx.x / LPR);
     const double* lam = a.lam_out + (uint64_t)(t + 1) * R;
     const int* rank = a.rank + (uint64_t)(t + 1) * (R + 1);
-    jacobi_row<LPR>(a.log + (uint64_t)(t + 1) * (jacobi_log_doubles(R) / 2), rank[R], R, i, threadIdx.x,
-                    [&](int v, double x) {
-                        if (i >= R) return;
-                        const int at = rank[v];
-                        const double l = lam[at];
-                        // W[u][R-1-v] = V[u][v] / sqrt(lam[v]) when lam[v] > 1e-8
-                        // (efficient_krp_sampler.hpp:126-138); E rows sqrt(mu) v,
-                        // clamped at 0
-                        if (gram) a.W[i * R + (R - 1 - at)] = l > 1e-8 ? x / sqrt(l) : 0.0;
-                        else a.E[(uint64_t)a.modes[t] * R2 + at * R + i] = x * sqrt(l > 0.0 ? l : 0.0);
-                    });
+    jacobi_row<LPR>(cm_log(a, t), rank[R], R, i, threadIdx.x, [&](int v, double x) {
+        if (i >= R) return;
+        const int at = rank[v];
+        const double l = lam[at];
+        // W[u][R-1-v] = V[u][v] / sqrt(lam[v]) when lam[v] > 1e-8
+        // (efficient_krp_sampler.hpp:126-138); E rows sqrt(mu) v, clamped at 0
+        if (gram) a.W[i * R + (R - 1 - at)] = l > 1e-8 ? x / sqrt(l) : 0.0;
+        else a.E[(uint64_t)a.modes[t] * R2 + at * R + i] = x * sqrt(l > 0.0 ? l : 0.0);
+    });
 }
 
 __global__ void __launch_bounds__(256) k_cm_pinv(ComputeMSel sel) {
