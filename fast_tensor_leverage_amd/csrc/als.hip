@@ -1095,14 +1095,6 @@ struct Als {
             lk->init(N, I, J, R, U, true, stream, kind == 2);
         } else {
             sampler = sampler_new_aliased(N, I, J, R, U, precision);
-            // after an update a factor is zero in all rows without a matched
-            // nonzero and dominated by a few heavy ones: most samples descend to
-            // nodes that the caches hold anyway, and the others' paths follow
-            // their uniforms less.  Per sweep: ordered 4,706-4,764, in tiles
-            // 4,838-4,853, plain 4,550-4,573 us at 2^20 x 2^19 x 2^15, 2e7
-            // nonzeros, R = 25; in tiles 5,091, plain 4,799 at 183 x 24 x 1140 x 1717.
-            sampler_set_option(sampler, "tile_descent", 0);
-            sampler_set_option(sampler, "sample_order", 0);
         }
         samples = mem.alloc<uint64_t>(N * J);
         FTL_HIP_CHECK(hipMemsetAsync(samples, 0, N * J * sizeof(uint64_t), stream));

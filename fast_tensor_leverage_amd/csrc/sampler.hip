@@ -365,6 +365,12 @@ constexpr uint64_t kOrderMaxJ = 1ull << 24;
 
 inline uint64_t order_blocks(uint64_t J) { return (J + order_share(J) - 1) / order_share(J); }
 
+// Scratch of the sort of `rows` orders: the bins, then the count table.
+inline uint64_t order_bin_bytes(uint64_t rows, uint64_t J) { return (rows * J * sizeof(uint16_t) + 255) / 256 * 256; }
+inline uint64_t order_scratch_bytes(uint64_t rows, uint64_t J) {
+    return order_bin_bytes(rows, J) + rows * order_blocks(J) * kOrderBins * sizeof(uint32_t);
+}
+
 // Every solve's log fits the eigen tree that k_cm_solve keeps it in.
 constexpr bool cm_logs_fit() {
     for (uint64_t R = kJacobiSplitR; R <= 128; R++)
@@ -453,8 +459,10 @@ struct Sampler {
     uint32_t tile_descent = 2;
     uint32_t* st_r = nullptr;
     double* st_s = nullptr;
-    uint16_t* order_bin = nullptr;
-    uint32_t *order_count = nullptr, *order_perm = nullptr;
+    // order_rows orders (one a mode, two for tiles) and the sort's scratch
+    uint64_t order_rows = 0;
+    uint32_t* order_perm = nullptr;
+    char* order_scratch = nullptr;
     double* h_state = nullptr;
     bool timing = false;
     // events of every timed call since the last read-out: {start, after
@@ -803,12 +811,15 @@ struct Sampler {
         } else if (key == "sample_order") {
             FTL_REQUIRE(value >= 0 && value <= 2, "sample_order must be 0, 1 or 2");
             sample_order = (uint32_t)value;
+            ensure_order();
         } else if (key == "tile_descent") {
             FTL_REQUIRE(value >= 0 && value <= 2, "tile_descent must be 0, 1 or 2");
             tile_descent = (uint32_t)value;
+            ensure_order();
         } else if (key == "xcd_buckets") {
             FTL_REQUIRE(value == 0 || value == 1, "xcd_buckets must be 0 or 1");
             sample_order = value ? 1 : 2;
+            ensure_order();
         } else if (key == "draw_kernel") {
             FTL_REQUIRE(value >= 0 && value <= 3, "draw_kernel must be 0, 1, 2 or 3");
             draw_kernel = (uint32_t)value;
@@ -1018,13 +1029,7 @@ struct Sampler {
         etree = msets[0].etree;
         lam = msets[0].lam;
         h_state = dalloc<double>(J * R);
-        if (J <= kOrderMaxJ) {
-            order_bin = dalloc<uint16_t>(2 * N * J);
-            order_perm = dalloc<uint32_t>(2 * N * J);
-            order_count = dalloc<uint32_t>(2 * N * order_blocks(J) * kOrderBins);
-            st_r = dalloc<uint32_t>(J);
-            st_s = dalloc<double>(J * 4);
-        }
+        ensure_order();
         trees_dirty = true;
         if (sync_end) FTL_HIP_CHECK(hipStreamSynchronize(stream));
     }
@@ -1039,11 +1044,13 @@ struct Sampler {
         while (rmax < R) rmax *= 2;
         const uint64_t pad = tri_size(rmax) + kTreePadExtra;
         size_t total = 0;
+        uint64_t tree_max = 0;
         for (uint32_t k = 0; k < N; k++) {
             ModeHost m;
             m.I = I[k];
             m.F = std::min<uint64_t>(R, I[k]);
             m.sh = make_shape(m.I, m.F);
+            tree_max = std::max<uint64_t>(tree_max, m.sh.node_count * ts64 * sizeof(double));
             const uint32_t depth = shape_depth(m.sh);
             uint32_t d64 = depth + 1;
             if (prec == FTL_FP32) d64 = std::max<uint32_t>(1, depth + 1 > fp32_lv ? depth + 1 - fp32_lv : 0);
@@ -1062,9 +1069,10 @@ struct Sampler {
                  up((uint64_t)(N + 1) * R * 8);
         if (R >= (uint64_t)kJacobiSplitR) total += up((N + 1) * (R + 1) * sizeof(int));
         total += up(J * R * 8);
-        if (J <= kOrderMaxJ)
-            total += up(2 * N * J * 2) + up(2 * N * J * 4) + up(2 * N * order_blocks(J) * kOrderBins * 4) + up(J * 4) +
-                     up(J * 4 * 8);
+        // packed draws (R <= 64) take no order
+        const uint64_t rows = R <= 64 ? 0 : default_orders(N, J, R, tree_max) * N;
+        if (rows) total += up(rows * J * 4);
+        if (rows > N) total += up(J * 4) + up(J * 4 * 8);
         return total;
     }
 
@@ -1309,16 +1317,16 @@ struct Sampler {
     // and R = 52 at J = 50,000 557 / 541 and 1,806 / 1,693, at J = 65536 653 / 677
     // and 2,127 / 2,142.  Never at R <= 21 (R = 20, J = 65536 535 / 504) nor R <=
     // 16, which leaves most of a block empty: 531 / 455 us.
-    bool tiles_pay() const {
+    static bool tiles_pay(uint64_t J, uint64_t R) {
         if (R > 64) return J >= 8192;
         if (R <= 27 || (R > 48 && R <= 56)) return R > 21 && J >= 65536;
         return J >= 32768;
     }
     bool tiled(const std::vector<int>& order) const {
-        if (!st_s || !mode_split || tile_descent == 0) return false;
+        if (order_rows < 2 * N || !st_s || !mode_split || tile_descent == 0) return false;
         for (int k : order)
             if (modes[k].sh.node_count >= (1ull << 31)) return false;
-        return tile_descent == 1 || tiles_pay();
+        return tile_descent == 1 || default_orders(N, J, R, tree_max()) == 2;
     }
 
     // One sampled mode: eigen rows, upper Gram levels, then the rest.
@@ -1364,13 +1372,55 @@ struct Sampler {
     // than the sort (15 us beside computeM) and the indirection may cost: I =
     // 2^14, R = 32 511 / 530; I = 2^18, R = 16, six modes 453 / 475, but 578 /
     // 570 a call when samplers alternate; I = 1000, R = 8 47 / 45.
-    bool order_pays() const {
-        if (J < 2048 || R <= 16) return false;
-        for (const ModeHost& m : modes)
-            if (m.sh.node_count * ts64 * sizeof(double) >= (16u << 20)) return true;
-        return false;
+    static bool order_pays(uint64_t J, uint64_t R, uint64_t tree_max) {
+        return J >= 2048 && R > 16 && tree_max >= (16u << 20);
     }
-    bool ordered() const { return order_perm && (sample_order == 1 || (sample_order == 2 && order_pays())); }
+    bool ordered() const {
+        return order_rows && (sample_order == 1 || (sample_order == 2 && order_pays(J, R, tree_max()) &&
+                                                    order_scratch_bytes(N, J) <= J * R * sizeof(double)));
+    }
+
+    uint64_t tree_max() const {
+        uint64_t b = 0;
+        for (const ModeHost& m : modes) b = std::max<uint64_t>(b, m.sh.node_count * ts64 * sizeof(double));
+        return b;
+    }
+
+    // Orders a mode that draws take by default: two with the tile kernels, else
+    // one or none.  None whose sort does not find room in h_state, which no draw
+    // kernel has written yet when it runs (N = 9 and more at R = 22; never at R >
+    // 64): memory for it could be more than a request's budget holds.
+    static uint64_t default_orders(uint64_t N, uint64_t J, uint64_t R, uint64_t tree_max) {
+        const uint64_t room = J * R * sizeof(double);
+        if (J > kOrderMaxJ) return 0;
+        if (tiles_pay(J, R) && order_scratch_bytes(2 * N, J) <= room) return 2;
+        return order_pays(J, R, tree_max) && order_scratch_bytes(N, J) <= room ? 1 : 0;
+    }
+
+    // Memory of the orders that the options ask for (none yet while the
+    // constructor applies the tuning table).
+    void ensure_order() {
+        if (!h_state || J > kOrderMaxJ) return;
+        const uint64_t by_rule = default_orders(N, J, R, tree_max());
+        const bool tiles = tile_descent == 1 || (tile_descent == 2 && by_rule == 2);
+        const uint64_t rows = tiles ? 2 * N : sample_order == 1 || (sample_order == 2 && by_rule) ? N : 0;
+        if (tiles && !st_s) {
+            st_r = dalloc<uint32_t>(J);
+            st_s = dalloc<double>(J * 4);
+        }
+        if (rows <= order_rows) return;
+        if (order_rows) {
+            FTL_HIP_CHECK(hipDeviceSynchronize());  // draws that read them
+            if (order_scratch != (char*)h_state) dfree(order_scratch, order_scratch_bytes(order_rows, J));
+            dfree(order_perm, order_rows * J * sizeof(uint32_t));
+            order_perm = nullptr;
+            order_rows = 0;
+        }
+        order_perm = dalloc<uint32_t>(rows * J);
+        const uint64_t scratch = order_scratch_bytes(rows, J);
+        order_scratch = scratch <= J * R * sizeof(double) ? (char*)h_state : dalloc<char>(scratch);
+        order_rows = rows;
+    }
 
     // The orders of every sampled mode's samples (k_order_*) by their Gram
     // uniforms and, with eigen, by their eigen uniforms, queued on st.
@@ -1384,10 +1434,11 @@ struct Sampler {
         o.seed = seed;
         o.call = call;
         o.share = order_share(J);
-        o.bin = order_bin;
-        o.count = order_count;
+        const unsigned rows = (unsigned)order.size() * (eigen ? 2 : 1);
+        o.bin = reinterpret_cast<uint16_t*>(order_scratch);
+        o.count = reinterpret_cast<uint32_t*>(order_scratch + order_bin_bytes(rows, J));
         o.perm = order_perm;
-        const dim3 grid((unsigned)order_blocks(J), (unsigned)order.size() * (eigen ? 2 : 1));
+        const dim3 grid((unsigned)order_blocks(J), rows);
         hipLaunchKernelGGL(k_order_count, grid, dim3(256), 0, st, o);
         FTL_HIP_CHECK(hipGetLastError());
         hipLaunchKernelGGL(k_order_scatter, grid, dim3(256), 0, st, o);
@@ -1581,6 +1632,8 @@ Sampler* sampler_new_async(uint32_t N, const uint64_t* I, uint64_t J, uint64_t R
                            DeviceAllocator* alloc, hipStream_t st) {
     std::unique_ptr<Sampler> s(new Sampler());
     s->allocator = alloc;
+    // up to R = 64 drawn packed, in index order
+    if (R <= 64) s->sample_order = s->tile_descent = 0;
     s->init(N, I, J, R, U_dev, true, precision, true, false, st);
     return s.release();
 }
@@ -1705,6 +1758,13 @@ size_t sampler_footprint(uint32_t N, const uint64_t* I, uint64_t J, uint64_t R, 
 Sampler* sampler_new_aliased(uint32_t N, const uint64_t* I, uint64_t J, uint64_t R, double* const* U_dev,
                              int precision) {
     std::unique_ptr<Sampler> s(new Sampler());
+    // after an update a factor is zero in all rows without a matched nonzero and
+    // dominated by a few heavy ones: most samples descend to nodes that the caches
+    // hold anyway, and the others' paths follow their uniforms less.  Per sweep:
+    // ordered 4,706-4,764, in tiles 4,838-4,853, plain 4,550-4,573 us at 2^20 x
+    // 2^19 x 2^15, 2e7 nonzeros, R = 25; in tiles 5,091, plain 4,799 at 183 x 24 x
+    // 1140 x 1717.
+    s->sample_order = s->tile_descent = 0;
     s->init(N, I, J, R, U_dev, true, precision, true);
     return s.release();
 }

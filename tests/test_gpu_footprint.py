@@ -27,7 +27,7 @@ def _blocks(dims, R, J, sets):
     return out + [8 * J * R, 8 * J * R, 32 * J, 4 * J, 4 * J, 36]
 
 
-SHAPES = [((70, 300, 64), 33, 64), ((500, 40), 40, 1), ((200, 200, 200, 200), 64, 700), ((65, 129, 70), 65, 300),
+SHAPES = [((1000, 1000, 1000, 1000), 8, 1), ((3000, 40), 16, 2000), ((65536, 70, 64), 25, 2048), ((70, 300, 64), 33, 64), ((500, 40), 40, 1), ((200, 200, 200, 200), 64, 700), ((65, 129, 70), 65, 300),
           ((300, 300, 300), 128, 1000)]
 
 
@@ -40,7 +40,8 @@ def test_sampler_memory(dims, R, J):
     assert s.info()["device_bytes"] <= sum(_blocks(dims, R, J, 2))
 
 
-@pytest.mark.parametrize("dims,R,J", [s for s in SHAPES if s[1] > 40] + [((70, 300, 64), 33, 4000)])
+@pytest.mark.parametrize("dims,R,J", [s for s in SHAPES if s[1] > 40] + [((70, 300, 64), 33, 4000),
+                                                                           ((5000, 3000), 16, 1)])
 def test_served_request_fits(dims, R, J):
     import fast_tensor_leverage_amd as ftl
     print(f"[gpu] served request {dims} R={R} J={J}", flush=True)
@@ -50,3 +51,25 @@ def test_served_request_fits(dims, R, J):
     srv = ftl.Server(budget, 1)
     got = srv.wait(srv.submit(list(dims), R, J, None, 5, "fp64"))
     assert all(got[k].max() < n for k, n in enumerate(dims))
+
+
+def test_order_memory_grows_with_the_options():
+    """A sampler whose default takes no order gets the memory for it when an
+    option asks, more when a second one does, and draws the same samples."""
+    import fast_tensor_leverage_amd as ftl
+    print("[gpu] memory of the sample orders", flush=True)
+    rng = np.random.default_rng(9)
+    dims, R, J = (3001, 1, 517), 12, 3000
+    s = ftl.Sampler([rng.standard_normal((n, R)) for n in dims], J, R)
+    draws = rng.random(2 * 3 * J)
+    out, held = [], []
+    for key, value in ((None, 0), ("sample_order", 1), ("tile_descent", 1), ("tile_descent", 0), ("sample_order", 2)):
+        if key:
+            s.set_option(key, value)
+        samples = np.zeros((3, J), dtype=np.uint64)
+        s.KRPDrawSamples(4, samples, draws)
+        out.append(samples)
+        held.append(s.info()["device_bytes"])
+    for a in out[1:]:
+        np.testing.assert_array_equal(out[0], a)
+    assert held[0] < held[1] < held[2] == held[3] == held[4]
