@@ -154,6 +154,9 @@ def tune_bucket(ftl, torch, dev, precision, rb, db, jb, steps, mismatch_bar, rou
     gen.manual_seed(5)
     draws = torch.rand(2 * N_MODES * J, generator=gen, device=dev, dtype=torch.float64)
     smp = ftl.Sampler.from_device(U, J, R, precision=precision)
+    # a row's kernel and launch shape are for the draws of its bucket that the
+    # tile kernels do not take: every candidate is timed without them
+    smp.set_option("tile_descent", 0)
     if "fp32_levels" in opts:
         smp.set_option("fp32_levels", opts["fp32_levels"])
     d_s = torch.zeros((N_MODES, J), dtype=torch.int64, device=dev)

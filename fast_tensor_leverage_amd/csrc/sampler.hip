@@ -449,6 +449,8 @@ struct Sampler {
     // 6.20 (128 threads) / 7.23 (256); R=128 group 172.5 ms (the 129
     // coefficients and node values per lane spill), block 27.8 (256 threads)
     uint32_t draw_kernel = 0;
+    // set_option chose it (a tuning row's choice is for draws without tiles)
+    bool kernel_asked = false;
     // threads per block of the one-sample-per-block kernel (0: by rank)
     uint32_t block_threads = 0;
     // option "sample_order": launches take the samples by increasing Gram
@@ -823,6 +825,7 @@ struct Sampler {
         } else if (key == "draw_kernel") {
             FTL_REQUIRE(value >= 0 && value <= 3, "draw_kernel must be 0, 1, 2 or 3");
             draw_kernel = (uint32_t)value;
+            kernel_asked = value != 0;
         } else if (key == "block_threads") {
             FTL_REQUIRE(value == 0 || value == 128 || value == 256 || value == 512,
                         "block_threads must be 0, 128, 256 or 512");
@@ -885,6 +888,7 @@ struct Sampler {
             } catch (const Error&) {
             }
         }
+        kernel_asked = false;
     }
 
     int64_t get_option(const std::string& key) const {
@@ -1326,7 +1330,12 @@ struct Sampler {
         if (order_rows < 2 * N || !st_s || !mode_split || tile_descent == 0) return false;
         for (int k : order)
             if (modes[k].sh.node_count >= (1ull << 31)) return false;
-        return tile_descent == 1 || default_orders(N, J, R, tree_max()) == 2;
+        if (tile_descent == 1) return true;
+        // not by rule against a kernel or a grid that the caller asked for; the
+        // kernels of the rank itself (2 above R = 64, 3 up to it) end the tiles
+        if (grid_override || (kernel_asked && (R <= 32 ? draw_kernel == 1 : R <= 64 ? draw_kernel == 2 : draw_kernel == 3)))
+            return false;
+        return default_orders(N, J, R, tree_max()) == 2;
     }
 
     // One sampled mode: eigen rows, upper Gram levels, then the rest.

@@ -190,8 +190,11 @@ void* ftl_sampler_stream(ftl_sampler* s);
  * the samples: 0 = by index, 1 = by Gram uniform, a contiguous part per XCD,
  * 2 = 1 where it pays, the default; J <= 2^24), "xcd_buckets" (1 sets
  * "sample_order" 1, 0 sets 2), "tile_descent" (eigen descents and upper Gram
- * levels of 16 ordered samples per wave on the FP64 matrix cores: 0 never,
- * 1 with "mode_split" and J <= 2^24, 2 = 1 where it pays, the default),
+ * levels of 16 ordered samples per wave on the FP64 matrix cores, the rest by
+ * the rank's kernel, "grid_blocks" capping that one's blocks: 0 never, 1 with
+ * "mode_split" and J <= 2^24 whatever "draw_kernel" says, 2, the default, where
+ * it pays, unless set_option gave "grid_blocks" or a "draw_kernel" other than
+ * the rank's; a tuning row's "draw_kernel" is for draws without tiles),
  * "overlap_compute_m" (1, the
  * default for a sampler with a stream of its own: computeM of a call runs on
  * a second stream into one of two buffer sets, overlapping the previous
