@@ -43,19 +43,6 @@ __device__ inline double fast_rsq(double x) {
     return fma(r, e, r);
 }
 
-// Pair k of round `round` in the circle-method ordering of n2 (even) indices:
-// position 0 fixed, positions 1..n2-1 rotating; returned with p < q.
-__device__ inline void jacobi_pair(int k, int round, int n2, int& p, int& q) {
-    p = k == 0 ? 0 : 1 + ((k - 1 + round) % (n2 - 1));
-    const int kk = n2 - 1 - k;
-    q = kk == 0 ? 0 : 1 + ((kk - 1 + round) % (n2 - 1));
-    if (p > q) {
-        const int t = p;
-        p = q;
-        q = t;
-    }
-}
-
 // The rotation of tangent t != 0.
 __device__ inline void jacobi_cs(double t, double& c, double& s) {
 #pragma clang fp contract(off)
@@ -97,8 +84,6 @@ __device__ inline bool jacobi_rotation(const double* A, int LD, int R, int p, in
     return jacobi_rotation(A[p * LD + p], A[q * LD + q], A[p * LD + q], c, s, t);
 }
 
-// Returns false (in every thread) when the sweep cap ended the iteration
-// before every pair met the skip test.
 // Sweep cap of the cyclic Jacobi iteration (quadratic convergence takes
 // 6-10 sweeps for R <= 128 in FP64).
 constexpr int kJacobiMaxSweeps = 40;
@@ -302,7 +287,8 @@ __device__ __forceinline__ int jacobi_open(const double* A, int LD, int R) {
 // its larger index only has the sign of its s turned.  k_gram_pinv over 700- and
 // 300-row Gaussian / ill-conditioned factors, two barriers a round -> this (us):
 // R = 32 156 / 296 -> 113 / 203, R = 16 59 / 123 -> 45 / 91.  Vout may be A1; A0 is
-// overwritten.
+// overwritten.  Returns false (in every thread) when the sweep cap ended the
+// iteration before every pair met the skip test.
 template <int BS>
 __device__ __forceinline__ bool jacobi_small(double* A0, double* A1, double* V, int R, double* lam, double* Vout,
                                              JacobiShared& js, double* diag_tmp) {
@@ -546,8 +532,8 @@ __device__ __forceinline__ bool jacobi_large(double* A, double* V, int R, double
     bool converged = false;
     for (int sweep = 0; sweep < kJacobiMaxSweeps; sweep++) {
         int any = 0;
-        // circle-method positions of pair tid (jacobi_pair), advanced by one
-        // (mod n2 - 1) per round instead of recomputed by division
+        // circle-method positions of pair tid's elements, advanced by one (mod
+        // n2 - 1) per round instead of recomputed by division
         int pa = tid - 1, pb = n2 - 2 - tid;
         for (int round = 0; round + 1 < n2; round++) {
             // rotations of this round, each computed once from the current A
@@ -647,8 +633,6 @@ __device__ __forceinline__ bool jacobi_large(double* A, double* V, int R, double
 // Storage of a block.  R <= kJacobiSmallR: both buffers of A, the second also
 // the eigenvectors, and V, all in LDS.  Above: A in LDS, V ((R+1) R) and the
 // eigenvectors (R^2) in the block's global scratch.
-constexpr int kJacobiThreads = 1024;
-
 __host__ __device__ inline uint64_t jacobi_lds_doubles(uint64_t R) {
     if (R > (uint64_t)kJacobiSmallR) return (R + 1) * R;
     const uint64_t n2 = (uint64_t)jacobi_n2((int)R);

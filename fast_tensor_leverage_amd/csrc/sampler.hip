@@ -1216,7 +1216,8 @@ struct Sampler {
     // registers.  Draws with the wider class and now (us): three modes of 2^20, J
     // = 50,000, R = 20 641 / 500; 2^18, J = 20,000, R = 36 557 / 479, R = 48 992 /
     // 574, R = 52 932 / 694; with the leaf rows' loads of leaf_row, 183 x 24 x 1140
-    // x 1717, J = 65,536, R = 25 567 / 405.
+    // x 1717, J = 65,536, R = 25 567 / 405.  (The same loads would also hold R =
+    // 22, 41, 49-50 and 57; those ends are not measured.)
     template <typename F>
     void with_cfg(F&& f) const {
         using std::integral_constant;

@@ -24,7 +24,7 @@ struct DeviceAllocator {
 Sampler* sampler_new_aliased(uint32_t N, const uint64_t* I, uint64_t J, uint64_t R, double* const* U_dev,
                              int precision);
 void sampler_delete(Sampler* s);
-// Same, allocating from `alloc` and leaving the tree builds queued on stream
+// Same, allocating from `alloc` (up to R = 64 for packed draws only) and leaving the tree builds queued on stream
 // `st` (borrowed; no host wait).
 Sampler* sampler_new_async(uint32_t N, const uint64_t* I, uint64_t J, uint64_t R, double* const* U_dev, int precision,
                            DeviceAllocator* alloc, hipStream_t st);
@@ -40,8 +40,9 @@ void sampler_rebuild(Sampler* s, uint32_t j, hipStream_t st);
 void sampler_set_seed(Sampler* s, uint64_t seed, uint64_t counter);
 // Packed draws (one launch of each computeM kernel and one of the draw
 // kernel for several samplers of the same R, precision and launch options,
-// each drawing all its sampled modes with its built-in uniforms; the samples
-// equal those of its own draw).  dev_args / host_stage hold
+// each drawing all its sampled modes with its built-in uniforms; the samples are
+// those of its own draw with "tile_descent" 0, bit for bit, and those of its own
+// draw through the tile kernels where no uniform is within rounding of a bound).  dev_args / host_stage hold
 // packed_args_bytes(n) bytes (host_stage pinned, reusable once the copy
 // queued on st has run); the samplers' trees must be complete in st's order.
 struct PackItem {

@@ -15,7 +15,9 @@
 // Samples of the tile that stand at different nodes are served one node after
 // the other.  Deep in the tree each sample stands alone and the group kernel is
 // the better one: a descent stops when a level took more than kTileStop nodes
-// and is resumed there.
+// and is resumed there.  With J samples in the order of their uniforms that is
+// about two levels past log2(J / 16): level 13.8 on average for J = 50,000, of 18
+// at I = 2^23, R = 32.
 #pragma once
 
 #include "sampler_kernels.hpp"
