@@ -188,7 +188,8 @@ void* ftl_sampler_stream(ftl_sampler* s);
  * "block_threads" (threads per block of the one-sample-per-block kernel:
  * 128/256/512, 0 = 256), "sample_order" (order in which the draw kernels take
  * the samples: 0 = by index, 1 = by Gram uniform, a contiguous part per XCD,
- * 2 = 1 where it pays, the default; J <= 2^24), "xcd_buckets" (1 sets
+ * 2 = 1 where it pays, the default; J <= 2^24; the first 1 that needs memory
+ * the sampler does not hold yet allocates it), "xcd_buckets" (1 sets
  * "sample_order" 1, 0 sets 2), "tile_descent" (eigen descents and upper Gram
  * levels of 16 ordered samples per wave on the FP64 matrix cores, the rest by
  * the rank's kernel, "grid_blocks" capping that one's blocks: 0 never, 1 with
